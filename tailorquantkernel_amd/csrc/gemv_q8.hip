@@ -421,52 +421,76 @@ size_t lds_bytes(int t, int nb, bool xf) {
 
 // ---------------------------------------------------------------------------
 // Many tokens: int8 MFMA GEMM.  A work-group of 8 waves computes a 128-row x
-// 128-token tile; wave w owns rows 32(w%4)..+31 (two 16-row tiles) of tokens
-// 64(w/4)..+63 (four 16-token tiles).  The K dimension goes 4 blocks (128
-// codes) per stage through two LDS buffers filled by direct-to-LDS copies, one
-// stage ahead of the one being multiplied; at 73.7 KB two work-groups share a
-// CU, so one's scaling overlaps the other's products.  Per block,
-// v_mfma_i32_16x16x32_i8 gives the exact int32 block dot for a 16 x 16 tile,
-// and each lane folds its four into fp32 with fma(s, w_d * x_d, acc): one
-// fp32 scaling per (row, token, block), the reference's per-block product
-// (kernel/q8_scalar.c:9-11) with one rounding fewer, summed over blocks in
-// order.
+// 128-token tile; wave w owns rows 32(w%4)..+31 of tokens 64(w/4)..+63, two
+// 32 x 32 tiles.  The K dimension goes 4 blocks (128 codes) per stage through
+// two LDS buffers filled by direct-to-LDS copies, one stage ahead of the one
+// being multiplied; at 74.8 KB and 128 registers two work-groups share a CU,
+// four waves per SIMD.
+//
+// Per block, v_mfma_i32_32x32x32_i8 (one 32-value block deep, the int8 form
+// that runs at the full 2,048 operations per cycle: 32 cycles for what four
+// 16x16x32 products take 64) gives the exact int32 block dots with the tokens
+// as rows, and each lane folds its 16 with fma(s, w_d * x_d, acc): the
+// reference's per-block product (kernel/q8_scalar.c:9-11) with one rounding
+// fewer, summed over blocks in order.  The products w_d * x_d of two blocks
+// come from one v_mfma_f32_32x32x1_2b_f32, an outer product of depth 1 and
+// so each product rounded once, like v_mul_f32: 32 cycles per block for 16
+// vector multiplies, and the operands are one scale per lane instead of 17.
+//
+// What bounds it: per 32 x 32 tile and block the matrix products (32 + 32
+// cycles) and 32 vector instructions (about 70 cycles at four waves), which
+// overlap little (an fp32 MFMA keeps the vector unit from issuing).  Without
+// the copies the loop is at that sum; the copies cost the rest, so their
+// shape matters: a wave's weight copy reads 64 contiguous bytes per row (four
+// lanes a row; one lane a row, 16 bytes every row pitch, cost 20 % more).
+// Against 16 x 16 products, vector scale multiplies and 16-byte row pieces
+// (8B shapes): MLP over 2,048 rows 1,267 -> 977 us, its Q4 form over 100 rows
+// 145 -> 104 us, the attention layer over 2,048 rows 452 -> 354 us, results
+// unchanged bit for bit.
 //
 // Tile order: work-groups are dealt to the 8 XCDs round-robin, so the grid is
 // laid out so that every token tile of one row tile runs on the same XCD
 // (work-group w: XCD w % 8, row tile 8 (w/8 / n_tt) + w % 8) and the tile's
 // 128 weight rows are read from HBM once into that XCD's L2.
 //
-// LDS per stage (36,864 B):
-//   A   [4 blocks][2 halves][128 rows][16 B]   weight codes, one copy per 16 B
-//   WD  [4 blocks][128 rows] fp32             weight scales
+// LDS per stage (37,376 B):
+//   A   [2 halves][128 rows][4 slots][16 B]   weight codes (Q4: one nibble run
+//       instead of two halves), block b of row r in slot gemm_slot(b, r)
+//   WD  [128 rows][4 blocks] fp32             weight scales
 //   B   [128 tokens][4 blocks x 36 B]         the tokens' block_q8, as stored:
 //       with 16-byte aligned rows and a block count that is a multiple of 4,
 //       a token's 144 bytes are nine 16-byte copies (three rounds of 512, the
 //       last round's surplus lanes, whole waves, issue none); otherwise 36
-//       dword copies per token.
+//       dword copies per token.  Or, from the split layout, codes
+//       [4 blocks][2 halves][128 tokens][16 B], then scales
+//       [4 blocks][128 + 32 tokens] fp32 (two blocks' rows in other banks).
 constexpr int kGemmThreads = 512;
 constexpr int kGemmRows = 128, kGemmToks = 128, kGemmKB = 4, kGemmBufs = 2;
 constexpr int kGemmA = kGemmKB * 2 * kGemmRows * 16;            // 16,384
 constexpr int kGemmWD = kGemmKB * kGemmRows * 4;                // 2,048
+constexpr int kGemmScaleRow = kGemmToks + 32;                   // floats between two blocks' token scales
 constexpr int kGemmBRow = kGemmKB * kBlockBytes;                // 144 bytes per token
-constexpr int kGemmB = kGemmToks * kGemmBRow;                   // 18,432
-constexpr int kGemmBChunks = kGemmB / 16;                       // 1,152 16-byte copies
+constexpr int kGemmBRows = kGemmToks * kGemmBRow;               // 18,432
+constexpr int kGemmBChunks = kGemmBRows / 16;                   // 1,152 16-byte copies
 constexpr int kGemmBRounds = (kGemmBChunks + kGemmThreads - 1) / kGemmThreads;   // 3
-constexpr int kGemmStage = kGemmA + kGemmWD + kGemmB;           // 36,864 (16-byte multiple)
-constexpr int kGemmBWords = kGemmB / 4;                         // 4,608 dword copies
-constexpr int kGemmXsCodes = kGemmKB * kQK * kGemmToks;          // 16,384: split-layout codes, then scales
-static_assert(kGemmXsCodes + kGemmKB * kGemmToks * 4 == kGemmB, "the split layout fills the token stage");
+constexpr int kGemmBWords = kGemmBRows / 4;                     // 4,608 dword copies
+constexpr int kGemmXsCodes = kGemmKB * kQK * kGemmToks;         // 16,384: split-layout codes, then scales
+constexpr int kGemmB = kGemmXsCodes + kGemmKB * kGemmScaleRow * 4;   // 18,944
+constexpr int kGemmStage = kGemmA + kGemmWD + kGemmB;           // 37,376
+static_assert(kGemmBRows <= kGemmB && kGemmStage % 16 == 0 && kGemmToks == kGemmRows, "stage layout");
 static_assert(kGemmBChunks % 64 == 0 && (kGemmBRounds - 1) * kGemmThreads < kGemmBChunks,
               "the last B round's copies past the tile are whole waves");
-static_assert(kGemmA / 16 % kGemmThreads == 0 && kGemmWD / 4 % kGemmThreads == 0 &&
+static_assert(kGemmA / 16 % kGemmThreads == 0 && kGemmKB * kGemmRows == kGemmThreads &&
               kGemmBWords % kGemmThreads == 0, "whole copy rounds per stage");
 
-__device__ __forceinline__ long lds_pair(const unsigned char *p) {
-    const uint32_t lo = *reinterpret_cast<const uint32_t *>(p);
-    const uint32_t hi = *reinterpret_cast<const uint32_t *>(p + 4);
-    return (long)(((unsigned long)hi << 32) | lo);
-}
+// Slot of a stage's block (0..3) in its row's 64 bytes of codes (its own
+// inverse): any 8 consecutive rows then hold a block in 8 different 16-byte
+// bank groups.
+__device__ __forceinline__ int gemm_slot(int blk, int row) { return blk ^ ((row >> 1) & 3); }
+
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
 
 // BX4: the activation rows are 16-byte aligned and nb % 4 == 0.
 // Q4: tiled Q4 matrices.  A holds [4 blocks][128 rows][16 B] nibble bytes (one
@@ -474,13 +498,14 @@ __device__ __forceinline__ long lds_pair(const unsigned char *p) {
 // 8 codes (low nibbles for k < 16, high for k >= 16), and the int32 products
 // are shifted back by 4 before scaling.
 template <bool BX4, bool Q4, bool UNI, bool XS>
-__global__ __launch_bounds__(512) void gemm_q8_kernel(GemvArgs a) {
+__global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
     static_assert(!UNI || BX4, "uniform copies need whole 16-byte stages");
     static_assert(!XS || UNI, "the split layout is copied from uniform bases");
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l16 = lane & 15, lg = lane >> 4;
+    const int l32 = lane & 31, hi = lane >> 5;
+    const int q4_shift = hi ? 0 : 4;
     const int cols = a.cols, nb = a.nb;
     const int n_tt = (a.n_tok + kGemmToks - 1) / kGemmToks;
     const int n_rt = (a.rows_total + kGemmRows - 1) / kGemmRows;
@@ -496,10 +521,14 @@ __global__ __launch_bounds__(512) void gemm_q8_kernel(GemvArgs a) {
     const int stages = (nb + kGemmKB - 1) / kGemmKB;
     const int st_begin = ks * stages / a.ksplit, st_end = (ks + 1) * stages / a.ksplit;
     const int wr = 32 * (wave & 3), wt = 64 * (wave >> 2);
+    // where this wave's 64 token scales of a stage go: block wave / 2, tokens 64 (wave & 1)..
+    const int sdst = 4 * (kGemmScaleRow * (wave >> 1) + 64 * (wave & 1));
 
-    // A chunk c = tid + 512 j -> (block c / 256, half (c / 128) & 1, row c % 128):
-    // row = tid % 128 for every j; WD dword c = tid -> (block c / 128, row c % 128).
-    const int my_row = tid & 127;
+    // A: thread tid copies 16 bytes of row tid / 4 (both halves of the block,
+    // slot tid % 4); WD: one row's four scales per lane (dwords: scale tid % 4
+    // of row tid / 4).
+    const int my_row = tid >> 2;
+    const int my_blk = gemm_slot(tid & 3, my_row);
     const unsigned char *wrow;
     const float *drow;
     {
@@ -521,28 +550,31 @@ __global__ __launch_bounds__(512) void gemm_q8_kernel(GemvArgs a) {
     // scalar base (segment, group, block, half) plus this lane's fixed row
     // offset, with no vector address arithmetic per stage.
     constexpr bool uni = UNI;
-    const unsigned char *useg = nullptr;   // the tile's segment: codes, then scales at uscale
+    const unsigned char *useg = nullptr;   // the rows' segment: codes, then scales at uscale
+    const unsigned char *uwd = nullptr;    // the same for this wave's scale rows
     size_t uscale = 0;
     uint32_t vrow = 0, vdrow = 0, vb[kGemmBRounds];
     if constexpr (uni) {
         const bool s0 = row0 < a.seg_end[0], s1 = !s0 && row0 < a.seg_end[1];
-        useg = s0 ? a.seg[0].w : (s1 ? a.seg[1].w : a.seg[2].w);
+        useg = uwd = s0 ? a.seg[0].w : (s1 ? a.seg[1].w : a.seg[2].w);
         int rows = s0 ? a.seg[0].rows : (s1 ? a.seg[1].rows : a.seg[2].rows);
-        int start = s0 ? 0 : (s1 ? a.seg_end[0] : a.seg_end[1]);
-        int r = row0 + my_row < a.rows_total ? row0 + my_row : a.rows_total - 1;
+        const int start = s0 ? 0 : (s1 ? a.seg_end[0] : a.seg_end[1]);
+        auto clamped = [&](int r) { return (row0 + r < a.rows_total ? row0 + r : a.rows_total - 1) - start; };
+        int r = clamped(my_row), rd = clamped(64 * (wave & 1) + lane);
         if (a.hq) {
             // paired tile rt: rows 64 rt.. of the gate matrix, then the same
-            // rows of the up matrix.  A wave's copies all lie in one half
-            // (row tid % 128 = 64 (wave & 1) + lane), so its base stays uniform.
-            useg = (wave & 1) ? a.seg[1].w : a.seg[0].w;
+            // rows of the up matrix.  A wave's code copies (16 rows) and its
+            // scale copies (64 rows) each lie in one of them.
+            useg = wave < 4 ? a.seg[0].w : a.seg[1].w;
+            uwd = (wave & 1) ? a.seg[1].w : a.seg[0].w;
             rows = a.seg[0].rows;
-            start = 0;
-            r = 64 * rt + lane;
+            r = 64 * rt + (my_row & 63);
+            rd = 64 * rt + lane;
         }
         const uint32_t rowb = Q4 ? (uint32_t)cols / 2 : (uint32_t)cols;
         uscale = (size_t)rows * rowb;
-        vrow = (uint32_t)(r - start) * rowb;
-        vdrow = (uint32_t)(r - start) * (uint32_t)nb * 4u;
+        vrow = (uint32_t)r * rowb + 16u * (uint32_t)my_blk;
+        vdrow = (uint32_t)rd * (uint32_t)nb * 4u;
         if constexpr (XS) {
             // every copy of this lane is for token 64 (wave & 1) + lane of the
             // tile: its 16-byte half-block and its scale in the block-major runs
@@ -582,17 +614,13 @@ __global__ __launch_bounds__(512) void gemm_q8_kernel(GemvArgs a) {
         const int g = b0 / kGroupBlocks, i0 = b0 - g * kGroupBlocks;
         const int n = nb - g * kGroupBlocks < kGroupBlocks ? nb - g * kGroupBlocks : kGroupBlocks;
         if (Q4) {
-            // chunk tid -> (block tid / 128, row tid % 128): the block is the wave's
-            dma16s(useg + 16 * (b0 + (wave >> 1)), vrow, buf + 16 * 64 * wave);
+            dma16s(useg + 16 * b0, vrow, buf + 16 * 64 * wave);
         } else {
 #pragma unroll
-            for (int j = 0; j < kGemmA / 16 / kGemmThreads; j++) {
-                const int c = 64 * wave + kGemmThreads * j;   // the wave's first chunk
-                const int blk = c >> 8, half = (c >> 7) & 1;
-                dma16s(useg + g * kGroupBytes + 16 * (i0 + blk) + (half ? 16 * n : 0), vrow, buf + 16 * c);
-            }
+            for (int half = 0; half < 2; half++)
+                dma16s(useg + g * kGroupBytes + 16 * (i0 + half * n), vrow, buf + 16 * (64 * wave + kGemmThreads * half));
         }
-        dma4s(useg + uscale + 4 * (b0 + (wave >> 1)), vdrow, buf + kGemmA + 4 * 64 * wave);
+        if (wave < 2) dma16s(uwd + uscale + 4 * b0, vdrow, buf + kGemmA + 16 * 64 * wave);
         if constexpr (XS) {
             // codes: chunk c -> (block c / 256, half (c / 128) & 1, token c % 128),
             // the same [block][half][row] 16-byte layout as the weights, one
@@ -606,7 +634,7 @@ __global__ __launch_bounds__(512) void gemm_q8_kernel(GemvArgs a) {
                        buf + kGemmA + kGemmWD + 16 * c);
             }
             dma4s(a.xq + (size_t)a.n_tok * cols + 4 * ((size_t)(b0 + (wave >> 1)) * a.n_tok + tok0),
-                  vb[1] - 4u * (uint32_t)tok0, buf + kGemmA + kGemmWD + kGemmXsCodes + 4 * 64 * wave);
+                  vb[1] - 4u * (uint32_t)tok0, buf + kGemmA + kGemmWD + kGemmXsCodes + sdst);
         } else {
 #pragma unroll
             for (int j = 0; j < kGemmBRounds; j++) {
@@ -624,25 +652,15 @@ __global__ __launch_bounds__(512) void gemm_q8_kernel(GemvArgs a) {
             return;
         }
         const int b0 = st * kGemmKB;
+        const int bw = b0 + my_blk < nb ? b0 + my_blk : nb - 1;
         if (Q4) {
-            // chunk tid -> (block tid / 128, row tid % 128)
-            const int blk = tid >> 7;
-            const int b = b0 + blk < nb ? b0 + blk : nb - 1;
-            dma16(wrow + 16 * b, buf + 16 * (tid - lane));
+            dma16(wrow + 16 * bw, buf + 16 * (tid - lane));
         } else {
 #pragma unroll
-            for (int j = 0; j < kGemmA / 16 / kGemmThreads; j++) {
-                const int c = tid + kGemmThreads * j;
-                const int blk = c >> 8, half = (c >> 7) & 1;
-                const int b = b0 + blk < nb ? b0 + blk : nb - 1;
-                dma16(wrow + tiled_offset(nb, b, 16 * half), buf + 16 * (c - lane));
-            }
+            for (int half = 0; half < 2; half++)
+                dma16(wrow + tiled_offset(nb, bw, 16 * half), buf + 16 * (tid - lane + kGemmThreads * half));
         }
-        {
-            const int blk = tid >> 7;
-            const int b = b0 + blk < nb ? b0 + blk : nb - 1;
-            dma4(drow + b, buf + kGemmA + 4 * (tid - lane));
-        }
+        dma4(drow + (b0 + (tid & 3) < nb ? b0 + (tid & 3) : nb - 1), buf + kGemmA + 4 * (tid - lane));
         if (BX4) {
             // the last round's copies past the tile are left out (whole waves)
 #pragma unroll
@@ -663,13 +681,9 @@ __global__ __launch_bounds__(512) void gemm_q8_kernel(GemvArgs a) {
         }
     };
 
-    float acc[2][4][4];
+    v16f acc[2];
 #pragma unroll
-    for (int r2 = 0; r2 < 2; r2++)
-#pragma unroll
-        for (int t4 = 0; t4 < 4; t4++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) acc[r2][t4][i] = 0.0f;
+    for (int t2 = 0; t2 < 2; t2++) acc[t2] = v16f(0.0f);
 
     // Two buffers (73.7 KB, so two work-groups share a CU): stage st+1 is
     // copied while stage st is multiplied.
@@ -680,84 +694,81 @@ __global__ __launch_bounds__(512) void gemm_q8_kernel(GemvArgs a) {
         __syncthreads();   // stage st is in LDS everywhere; stage st-1's buffer is free
         if (st + 1 < st_end) issue(st + 1, smem + ((st + 1 - st_begin) & 1) * kGemmStage);
         const unsigned char *A = buf, *WD = buf + kGemmA, *B = buf + kGemmA + kGemmWD;
-        // two blocks at a time: the second block's LDS reads and products
-        // overlap the first one's scaling
-#pragma unroll 2
-        for (int blk = 0; blk < kGemmKB; blk++) {
-            // (with 16-byte token rows every stage is whole)
-            const bool valid = BX4 || st * kGemmKB + blk < nb;
-            long av[2], bv[4];
-            float wd[2][4], xd[4];
+        // the row's four scales (times 1/16 for the Q4 codes, which come as 16 x code)
+        float4 wd4 = *reinterpret_cast<const float4 *>(WD + (wr + l32) * 16);
+        if (Q4) wd4 = make_float4(wd4.x * 0.0625f, wd4.y * 0.0625f, wd4.z * 0.0625f, wd4.w * 0.0625f);
 #pragma unroll
-            for (int r2 = 0; r2 < 2; r2++) {
-                const int row = wr + 16 * r2;
-                if (Q4) {
-                    const long raw = lds_pair(A + ((blk * kGemmRows) + row + l16) * 16 + 8 * (lg & 1));
-                    const uint32_t w0 = (uint32_t)raw, w1 = (uint32_t)((unsigned long)raw >> 32);
-                    const uint32_t c0 = lg < 2 ? q4_lo16(w0) : q4_hi16(w0);
-                    const uint32_t c1 = lg < 2 ? q4_lo16(w1) : q4_hi16(w1);
-                    av[r2] = (long)(((unsigned long)c1 << 32) | c0);
-                } else {
-                    av[r2] = lds_pair(A + (((blk * 2 + (lg >> 1)) * kGemmRows) + row + l16) * 16 + 8 * (lg & 1));
-                }
-                const float4 w4 = *reinterpret_cast<const float4 *>(WD + (blk * kGemmRows + row + 4 * lg) * 4);
-                wd[r2][0] = w4.x; wd[r2][1] = w4.y; wd[r2][2] = w4.z; wd[r2][3] = w4.w;
-            }
+        for (int b2 = 0; b2 < kGemmKB; b2 += 2) {
+            // both blocks' scales: lane (l32, hi) holds those of block b2 + hi
+            const float wd = b2 == 0 ? (hi ? wd4.y : wd4.x) : (hi ? wd4.w : wd4.z);
+            float xd[2];
 #pragma unroll
-            for (int t4 = 0; t4 < 4; t4++) {
+            for (int t2 = 0; t2 < 2; t2++) {
+                const int t = wt + 32 * t2 + l32;
                 if constexpr (XS) {
-                    // 8-byte reads of 16-byte rows: no bank conflicts, as for A
-                    bv[t4] = lds_pair(B + ((blk * 2 + (lg >> 1)) * kGemmToks + wt + 16 * t4 + l16) * 16 + 8 * (lg & 1));
-                    xd[t4] = *reinterpret_cast<const float *>(B + kGemmXsCodes + (blk * kGemmToks + wt + 16 * t4 + l16) * 4);
+                    xd[t2] = *reinterpret_cast<const float *>(B + kGemmXsCodes + ((b2 + hi) * kGemmScaleRow + t) * 4);
                 } else {
-                    const unsigned char *tb = B + (wt + 16 * t4 + l16) * kGemmBRow + blk * kBlockBytes;
-                    bv[t4] = lds_pair(tb + 4 + 8 * lg);
-                    // the staged scale is always a real block's (past nb the copies
-                    // repeat block nb-1): load it unconditionally and select, so no
-                    // branch splits the block's LDS reads from its products
-                    const float xv = *reinterpret_cast<const float *>(tb);
-                    xd[t4] = valid ? xv : 0.0f;
+                    // (with 16-byte token rows every stage is whole; past nb the
+                    // copies repeat block nb - 1: load and select, no branch)
+                    const float xv = *reinterpret_cast<const float *>(B + t * kGemmBRow + (b2 + hi) * kBlockBytes);
+                    xd[t2] = BX4 || st * kGemmKB + b2 + hi < nb ? xv : 0.0f;
                 }
             }
-            // all eight products first, so that each one's latency hides
-            // under the others before its results are read
-            v4i c[2][4];
+            v4i wv[2], xv[2][2];
 #pragma unroll
-            for (int r2 = 0; r2 < 2; r2++)
+            for (int j = 0; j < 2; j++) {
+                const int blk = b2 + j;
+                if (Q4) {
+                    const u32x4 w = *reinterpret_cast<const u32x4 *>(A + ((wr + l32) * kGemmKB + gemm_slot(blk, wr + l32)) * 16);
 #pragma unroll
-                for (int t4 = 0; t4 < 4; t4++)
-                    c[r2][t4] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[r2], bv[t4], v4i{0, 0, 0, 0}, 0, 0, 0);
+                    for (int i = 0; i < 4; i++) wv[j][i] = (int)(((w[i] ^ 0x88888888u) << q4_shift) & 0xF0F0F0F0u);
+                } else {
+                    wv[j] = *reinterpret_cast<const v4i *>(
+                        A + ((hi * kGemmRows + wr + l32) * kGemmKB + gemm_slot(blk, wr + l32)) * 16);
+                }
 #pragma unroll
-            for (int r2 = 0; r2 < 2; r2++)
+                for (int t2 = 0; t2 < 2; t2++) {
+                    const int t = wt + 32 * t2 + l32;
+                    if constexpr (XS) {
+                        xv[j][t2] = *reinterpret_cast<const v4i *>(B + ((blk * 2 + hi) * kGemmToks + t) * 16);
+                    } else {
+                        const int *x = reinterpret_cast<const int *>(B + t * kGemmBRow + blk * kBlockBytes + 4 + 16 * hi);
+                        xv[j][t2] = v4i{x[0], x[1], x[2], x[3]};
+                    }
+                }
+            }
 #pragma unroll
-                for (int t4 = 0; t4 < 4; t4++)
+            for (int t2 = 0; t2 < 2; t2++) {
+                const v32f p = __builtin_amdgcn_mfma_f32_32x32x1f32(xd[t2], wd, v32f(0.0f), 0, 0, 0);
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        acc[r2][t4][i] = fmaf((float)(Q4 ? c[r2][t4][i] >> 4 : c[r2][t4][i]), wd[r2][i] * xd[t4],
-                                              acc[r2][t4][i]);
+                for (int j = 0; j < 2; j++) {
+                    const v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(xv[j][t2], wv[j], v16i(0), 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[t2][i] = fmaf((float)c[i], p[16 * j + i], acc[t2][i]);
+                }
+            }
         }
     }
 
-    // y[t][r]: lane (l16, lg) holds rows 4lg..4lg+3 of each 16-row tile for
-    // token l16 of each 16-token tile.  A split writes its partial instead.
+    // y[t][r]: lane (l32, hi) holds row l32 of the wave's 32, register i token
+    // 8 (i / 4) + 4 hi + i % 4 of each 32-token tile, so a store covers 32
+    // consecutive rows of two tokens.  A split writes its partial instead.
+    auto tok = [&](int t2, int i) { return wt + 32 * t2 + 8 * (i >> 2) + 4 * hi + (i & 3); };
     if (UNI && XS && a.hq) {
         // the paired tile's gate (rows 0-63) and up (rows 64-127) values meet
-        // in LDS as [token][row] with 132-float token rows (a float4 store of
-        // 16 tokens then covers all 64 banks); then h = silu(g) * u of the
-        // tile's two 32-row blocks, quantized as silu_quant8_kernel does, 8
-        // lanes x 4 values per (block, token), written in the split layout
-        // (codes of block b, token t at ((2b + half) n + t) 16, scales [b][t]
-        // after the n * inter code bytes)
+        // in LDS as [token][row] with 132-float token rows; then
+        // h = silu(g) * u of the tile's two 32-row blocks, quantized as
+        // silu_quant8_kernel does, 8 lanes x 4 values per (block, token),
+        // written in the split layout (codes of block b, token t at
+        // ((2b + half) n + t) 16, scales [b][t] after the n * inter code bytes)
         constexpr int kHs = kGemmRows + 4;
         static_assert(kGemmToks * kHs * 4 <= kGemmBufs * kGemmStage, "the fp32 tile fits the stage buffers");
         float *hs = reinterpret_cast<float *>(smem);
         __syncthreads();   // every wave is done with the last stage
 #pragma unroll
-        for (int r2 = 0; r2 < 2; r2++)
+        for (int t2 = 0; t2 < 2; t2++)
 #pragma unroll
-            for (int t4 = 0; t4 < 4; t4++)
-                *reinterpret_cast<float4 *>(hs + (wt + 16 * t4 + l16) * kHs + wr + 16 * r2 + 4 * lg) =
-                    make_float4(acc[r2][t4][0], acc[r2][t4][1], acc[r2][t4][2], acc[r2][t4][3]);
+            for (int i = 0; i < 16; i++) hs[tok(t2, i) * kHs + wr + l32] = acc[t2][i];
         __syncthreads();
         const int n = a.n_tok, inter = a.seg[0].rows;
         float *scales = reinterpret_cast<float *>(a.hq + (size_t)n * inter);
@@ -778,38 +789,25 @@ __global__ __launch_bounds__(512) void gemm_q8_kernel(GemvArgs a) {
         }
         return;
     }
+    const int r = row0 + wr + l32;
+    if (r >= a.rows_total) return;
+    float *y;
+    int ldy;
     if (a.ksplit > 1) {
-        float *p = a.part + (size_t)ks * a.n_tok * a.rows_total;
-#pragma unroll
-        for (int r2 = 0; r2 < 2; r2++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int r = row0 + wr + 16 * r2 + 4 * lg + i;
-#pragma unroll
-                for (int t4 = 0; t4 < 4; t4++) {
-                    const int t = tok0 + wt + 16 * t4 + l16;
-                    if (r < a.rows_total && t < a.n_tok) p[(size_t)t * a.rows_total + r] = acc[r2][t4][i];
-                }
-            }
-        return;
+        y = a.part + (size_t)ks * a.n_tok * a.rows_total + r;
+        ldy = a.rows_total;
+    } else {
+        const bool s0 = r < a.seg_end[0], s1 = !s0 && r < a.seg_end[1];
+        y = (s0 ? a.seg[0].y : (s1 ? a.seg[1].y : a.seg[2].y)) + (r - (s0 ? 0 : (s1 ? a.seg_end[0] : a.seg_end[1])));
+        ldy = s0 ? a.seg[0].rows : (s1 ? a.seg[1].rows : a.seg[2].rows);
     }
 #pragma unroll
-    for (int r2 = 0; r2 < 2; r2++) {
+    for (int t2 = 0; t2 < 2; t2++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int r = row0 + wr + 16 * r2 + 4 * lg + i;
-            if (r >= a.rows_total) continue;
-            const bool s0 = r < a.seg_end[0], s1 = !s0 && r < a.seg_end[1];
-            float *y = s0 ? a.seg[0].y : (s1 ? a.seg[1].y : a.seg[2].y);
-            const int rows = s0 ? a.seg[0].rows : (s1 ? a.seg[1].rows : a.seg[2].rows);
-            const int lr = r - (s0 ? 0 : (s1 ? a.seg_end[0] : a.seg_end[1]));
-#pragma unroll
-            for (int t4 = 0; t4 < 4; t4++) {
-                const int t = tok0 + wt + 16 * t4 + l16;
-                if (t < a.n_tok) y[(size_t)t * rows + lr] = acc[r2][t4][i];
-            }
+        for (int i = 0; i < 16; i++) {
+            const int t = tok0 + tok(t2, i);
+            if (t < a.n_tok) y[(size_t)t * ldy] = acc[t2][i];
         }
-    }
 }
 
 // The split-K sum: y of (token t, row r) is the splits' partials added in

@@ -211,6 +211,22 @@ def test_gemm_vs_oracle(nat, oracle, rows, cols, n_tok, monkeypatch):
     check_matmul(gpu_matmul(nat, M, xq, n_tok), ref, Wq, xq, rows, cols, n_tok, f"default {rows}x{cols} n_tok={n_tok}")
 
 
+@pytest.mark.parametrize("rows,n_tok", [(1, 1), (31, 33), (32, 32), (33, 31), (97, 65), (129, 127), (160, 129)])
+@pytest.mark.parametrize("cols", [32, 128, 160, 2176])
+def test_gemm_tile_edges(nat, oracle, rows, n_tok, cols, monkeypatch):
+    """The GEMM at the edges of its 32 x 32 tiles and 4-block stages (2176: a
+    second 64-block group of 4), with scales that differ per block by orders
+    of magnitude, so a scale taken from another block, row or token shows."""
+    monkeypatch.setenv("TQ_HIP_GEMM_MIN_TOKENS", "1")
+    Wq = random_weights(oracle, rows, cols, rows + cols)
+    xq = quantize_tokens(oracle, fill_random(n_tok * cols, 5 * rows + cols, 1.0), n_tok, cols)
+    rng = np.random.default_rng(rows * n_tok + cols)
+    Wq["d"] *= 10.0 ** rng.uniform(-2, 2, Wq["d"].shape).astype(np.float32)
+    xq["d"] *= 10.0 ** rng.uniform(-2, 2, xq["d"].shape).astype(np.float32)
+    y = gpu_matmul(nat, Matrix(nat, Wq, rows, cols), xq, n_tok)
+    check_matmul(y, oracle.matmul_q8(Wq, xq, rows, cols, n_tok), Wq, xq, rows, cols, n_tok, (rows, cols, n_tok))
+
+
 @pytest.mark.parametrize("rw", ["1", "2", "4"])
 def test_rows_per_wave_identical(nat, oracle, rw, monkeypatch):
     """The rows-per-wave choice changes the launch shape, not one bit of the result."""
