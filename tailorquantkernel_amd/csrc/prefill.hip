@@ -43,25 +43,24 @@
 //   B operand of the P.V product (keys permuted identically in A and B), so P
 //   never goes through LDS.
 //
-// Balance: under the causal mask query block b reads b + 1 key tiles.  Two
-// attention kernels share the per-tile code:
+// Balance: under the causal mask query block b reads b + 1 key tiles.
+// prefill_block_kernel runs one work-group of 8 waves per (query block, kv
+// head), dealt longest block first, so the CUs pair long blocks with short
+// ones by themselves.  Its two 4-wave halves cover the same 128 rows and split
+// the block's key tiles (half h: tiles h, h+2, ...), then merge through LDS in
+// half order, each half finishing one row tile per wave.  Where the blocks
+// leave CUs idle they are cut into runs of tiles, one work-group each: each
+// writes its merged partial (o, m, l per row) with agent-coherent 16-byte
+// stores, waits for them and arrives on a counter; the last to arrive merges
+// the partials in run order, so the result does not depend on which finished
+// last.  No work-group waits on another.
 //
-// prefill_block_kernel — with at least two query blocks per CU (the 2048-
-//   token prefill: 64 blocks x 8 kv heads), one work-group of 8 waves per
-//   (query block, kv head), dealt longest block first, so the CUs pair long
-//   blocks with short ones by themselves.  Its two 4-wave halves cover the
-//   same 128 rows and split the block's key tiles (half h: tiles h, h+2, ...);
-//   half 1 leaves its (o, m, l) in LDS and half 0 merges the two in half
-//   order.  Nothing leaves the work-group but the output rows.
-// prefill_kernel — with fewer blocks, query blocks are paired last with first
-//   (p with nb-1-p), so every pair reads about the same number of tiles, and a
-//   pair's tile sequence (the later block's tiles, then the earlier block's)
-//   is cut into nsp equal chunks, one 4-wave work-group each.  A block covered
-//   by several segments: every segment writes its partial (o, m, l per row)
-//   with agent-coherent 16-byte stores, waits for them and arrives on a
-//   counter; the last to arrive merges the partials and its own registers in
-//   segment order, so the result does not depend on which finished last.  No
-//   work-group waits on another.
+// Halves merged in LDS before anything leaves the work-group is what makes
+// short prompts cheap: 4-wave segments of paired blocks, each writing its own
+// partial (up to 8 per block, read back one after the other), took 31 us where
+// this takes 24 (300 tokens, 32 / 8 heads of 128, staging launch included),
+// 58 -> 46 for 333 tokens after 1,000, 115 -> 67 for 1,500 tokens and
+// 142 -> 74 for 100 tokens after 8,000.
 //
 // Grid: one dimension, work-group w serves kv head w % n_kv, so with 8 kv
 // heads each XCD (work-groups go round-robin over the 8 XCDs) works on one
@@ -82,8 +81,11 @@ constexpr int kKT = 32;                  // keys per tile
 constexpr int kMaxPrefillKeys = 65536;   // keys [0, kend) the dense path serves
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.0f;            // log2 headroom before the running max moves
-constexpr int kMaxSplitsP = 8;           // chunks of one query-block pair
-constexpr int kItemOverheadTiles = 3;    // prologue + merge of a work item, in tile times
+constexpr int kMaxRuns = 8;              // runs of one query block
+// The plan's costs, in steps (a pair of key tiles, about 1.7 us at head_dim
+// 128): a work-group's prologue and store, its partial, and each run the last
+// one merges.
+constexpr double kItemCost = 3.5, kRunCost = 1.5, kMergeCost = 0.5;
 constexpr int kCounterStrideP = 64;      // ints: one 256-byte line per counter
 constexpr int kCoherentP = 16;           // cache policy sc1: agent-coherent access
 
@@ -518,7 +520,8 @@ struct PrefillArgs {
     int pos0;
     int n;
     int qblocks;         // query blocks of QB tokens
-    int nsp;             // chunks per block pair = most segments of one block
+    int chunk;           // key tiles per run of a block (0: every block is one run)
+    int nsp;             // most runs of one block
     int n_kv;
     float *partials;     // [n_kv][qblocks][nsp][RW][HD + 4]
     int *counters;       // [n_kv][qblocks] x kCounterStrideP
@@ -537,6 +540,9 @@ __host__ __device__ inline int block_tiles(int pos0, int n, int qb, int b) {
     const int last = (b + 1) * qb < n ? (b + 1) * qb : n;
     return (pos0 + last + kKT - 1) / kKT;
 }
+
+// Runs a block of nt tiles is cut into.
+__host__ __device__ inline int block_runs(int nt, int chunk) { return chunk == 0 ? 1 : (nt + chunk - 1) / chunk; }
 
 // Per-row state of one wave's NJ row tiles over a run of key tiles: o and
 // lsum are taken against moff (mrow, or 0 before any key); mrow is the running
@@ -737,14 +743,17 @@ __device__ __forceinline__ void tile_update(const PrefillArgs &a, const unsigned
     tile_pv<HD, G, NJ>(T, lane, pp, st);
 }
 
-// Normalise and store the wave's rows: lane holds columns 16m + 4lg .. +3 of
-// query l16.  Either fp32 rows into out, or (out_xs) each row quantized as
+// Normalise and store row tile nt (16 rows): lane holds columns
+// 16m + 4lg .. +3 of query l16.  Either fp32 rows into out, or (out_xs) each row quantized as
 // quantize_row_q8 straight into the split layout the output GEMM reads.
 template <int HD, int G, int NJ>
-__device__ __forceinline__ void store_rows(const PrefillArgs &a, int kvh, int i0, int wave, int lane,
-                                           const PRows<HD, G, NJ> &st, const float (&lrow)[NJ]) {
+__device__ __forceinline__ void store_rows(const PrefillArgs &a, int kvh, int i0, int nt, int lane,
+                                           const v4f (&o)[HD / 16], float lrow) {
     using S = PShape<HD, G, NJ>;
     const int l16 = lane & 15, lg = lane >> 4;
+    const float inv = 1.0f / lrow;
+    const int g = nt / S::QT;
+    const int qi = i0 + (nt % S::QT) * 16 + l16;
     if (a.out_xs) {
         // block b of a head is columns 32b..32b+31, tiles m = 2b (codes 0-15)
         // and 2b+1 (codes 16-31), 8 values in each of the 4 lanes of the
@@ -754,62 +763,49 @@ __device__ __forceinline__ void store_rows(const PrefillArgs &a, int kvh, int i0
         const size_t nrows = (size_t)a.n, cols = (size_t)a.n_q_heads * HD;
         float *xd = reinterpret_cast<float *>(a.out_xs + nrows * cols);
 #pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            const float inv = 1.0f / lrow[j];
-            const int nt = wave * NJ + j;
-            const int g = nt / S::QT;
-            const int qi = i0 + (nt % S::QT) * 16 + l16;
+        for (int b = 0; b < HD / kQK; b++) {
+            const v4f x0 = o[2 * b] * inv, x1 = o[2 * b + 1] * inv;
+            float m = 0.0f;
 #pragma unroll
-            for (int b = 0; b < HD / kQK; b++) {
-                const v4f x0 = st.o[2 * b][j] * inv, x1 = st.o[2 * b + 1][j] * inv;
-                float m = 0.0f;
+            for (int i = 0; i < 4; i++) {
+                const float a0 = x0[i] < 0.0f ? -x0[i] : x0[i];
+                const float a1 = x1[i] < 0.0f ? -x1[i] : x1[i];
+                m = fmaxf(m, a0 > 0.0f ? a0 : 0.0f);
+                m = fmaxf(m, a1 > 0.0f ? a1 : 0.0f);
+            }
+            m = fmaxf(m, __shfl_xor(m, 16));
+            m = fmaxf(m, __shfl_xor(m, 32));
+            const float d = quant_scale(m);
+            const float qinv = quant_inverse(d);
+            uint32_t w0 = 0, w1 = 0;
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float a0 = x0[i] < 0.0f ? -x0[i] : x0[i];
-                    const float a1 = x1[i] < 0.0f ? -x1[i] : x1[i];
-                    m = fmaxf(m, a0 > 0.0f ? a0 : 0.0f);
-                    m = fmaxf(m, a1 > 0.0f ? a1 : 0.0f);
-                }
-                m = fmaxf(m, __shfl_xor(m, 16));
-                m = fmaxf(m, __shfl_xor(m, 32));
-                const float d = quant_scale(m);
-                const float qinv = quant_inverse(d);
-                uint32_t w0 = 0, w1 = 0;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    w0 |= quant_code(x0[i], qinv) << (8 * i);
-                    w1 |= quant_code(x1[i], qinv) << (8 * i);
-                }
-                if (qi < a.n) {
-                    const size_t gb = (size_t)(kvh * G + g) * (HD / kQK) + b;
-                    *reinterpret_cast<uint32_t *>(a.out_xs + ((2 * gb) * nrows + qi) * 16 + 4 * lg) = w0;
-                    *reinterpret_cast<uint32_t *>(a.out_xs + ((2 * gb + 1) * nrows + qi) * 16 + 4 * lg) = w1;
-                    if (lg == 0) xd[gb * nrows + qi] = d;
-                }
+            for (int i = 0; i < 4; i++) {
+                w0 |= quant_code(x0[i], qinv) << (8 * i);
+                w1 |= quant_code(x1[i], qinv) << (8 * i);
+            }
+            if (qi < a.n) {
+                const size_t gb = (size_t)(kvh * G + g) * (HD / kQK) + b;
+                *reinterpret_cast<uint32_t *>(a.out_xs + ((2 * gb) * nrows + qi) * 16 + 4 * lg) = w0;
+                *reinterpret_cast<uint32_t *>(a.out_xs + ((2 * gb + 1) * nrows + qi) * 16 + 4 * lg) = w1;
+                if (lg == 0) xd[gb * nrows + qi] = d;
             }
         }
         return;
     }
+    if (qi < a.n) {
+        float *orow = a.out + ((size_t)qi * a.n_q_heads + (size_t)kvh * G + g) * HD;
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const float inv = 1.0f / lrow[j];
-        const int nt = wave * NJ + j;
-        const int g = nt / S::QT;
-        const int qi = i0 + (nt % S::QT) * 16 + l16;
-        if (qi < a.n) {
-            float *orow = a.out + ((size_t)qi * a.n_q_heads + (size_t)kvh * G + g) * HD;
-#pragma unroll
-            for (int m = 0; m < S::MT; m++) *reinterpret_cast<v4f *>(orow + m * 16 + 4 * lg) = st.o[m][j] * inv;
-        }
+        for (int m = 0; m < S::MT; m++) *reinterpret_cast<v4f *>(orow + m * 16 + 4 * lg) = o[m] * inv;
     }
 }
 
-// Merge the partial (ms, ls, os) into the running (M, L, acc), in order.
+// Merge the partial (ms, ls, os) into the running (M, L, acc), in order.  A
+// part that saw no key (m = -inf) adds nothing, whatever the other holds.
 template <int MT>
 __device__ __forceinline__ void merge_part(float &M, float &L, v4f (&acc)[MT], float ms, float ls, const v4f (&os)[MT]) {
     const float Mn = fmaxf(M, ms);
-    const float fo = __builtin_amdgcn_exp2f(M - Mn);   // 0 while M is -inf
-    const float fs = __builtin_amdgcn_exp2f(ms - Mn);  // 0 for a partial with no key
+    const float fo = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mn);
+    const float fs = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - Mn);
 #pragma unroll
     for (int m = 0; m < MT; m++) acc[m] = acc[m] * fo + os[m] * fs;
     L = L * fo + ls * fs;
@@ -836,177 +832,53 @@ __device__ __forceinline__ bool tile_has_rem(int gwave) {
     return I::REM > 0 && 64 * gwave < I::REM;
 }
 
-// One segment: query block blk against key tiles [kt_begin, kt_end), the
-// segment sp of the nsp that cover the block (4-wave work-group).
-template <int HD, int G, int NJ>
-__device__ __forceinline__ void prefill_segment(const PrefillArgs &a, int kvh, int blk, int kt_begin, int kt_end,
-                                                int sp, int nsp, unsigned char *tile0, unsigned char *tile1) {
-    using S = PShape<HD, G, NJ>;
-    using I = TileImg<HD>;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int l16 = lane & 15;
-    const int lg = lane >> 4;
-    const int i0 = blk * S::QB;
-    const unsigned char *img = a.img + (size_t)kvh * a.n_tiles * I::BYTES;
-
-    // ---- the block's staged q rows (prefill_stage_kernel) into tile1, then
-    //      the first key tile into tile0; waiting for all but this wave's
-    //      copies of the tile leaves only the tile in flight
-    {
-        constexpr int QCH = S::Q_BYTES / 16;
-        const unsigned char *src = a.qimg + ((size_t)kvh * a.qblocks + blk) * S::Q_BYTES;
-        const int wu = __builtin_amdgcn_readfirstlane(wave);
-        for (int c0 = 64 * wu; c0 < QCH; c0 += kThreads)
-            if (c0 + lane < QCH) dma16(src + 16 * (c0 + lane), tile1 + 16 * c0);
-    }
-    fetch_tile<HD>(img, kt_begin, tile0, tid, wave);
-    if (tile_has_rem<HD>(wave))
-        wait_vm<I::ROUNDS + 1>();
-    else
-        wait_vm<I::ROUNDS>();
-    __syncthreads();
-
-    PQ<HD, G, NJ> q;
-    load_q<HD, G, NJ>(a, tile1, i0, wave, lane, q);
-    PRows<HD, G, NJ> st;
-    st.init();
-
-    // ---- the key loop: two LDS buffers, one tile ahead, one barrier per tile
-    for (int kt = kt_begin; kt < kt_end; kt++) {
-        const bool odd = (kt - kt_begin) & 1;
-        unsigned char *T = odd ? tile1 : tile0;
-        // this thread's copies of tile kt have landed; the barrier makes every
-        // thread's visible and frees the other buffer (tile kt-1, or the q
-        // staging) for the next copy
-        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-        __syncthreads();
-        if (kt + 1 < kt_end) fetch_tile<HD>(img, kt + 1, odd ? tile0 : tile1, tid, wave);
-        tile_update<HD, G, NJ>(a, T, kt, i0, lane, q, st);
-    }
-
-    float lrow[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; j++) lrow[j] = xrow_sum(st.lsum[j]);
-    if (nsp == 1) {
-        store_rows<HD, G, NJ>(a, kvh, i0, wave, lane, st, lrow);
-        return;
-    }
-
-    // ---- split: every segment writes its partial rows [RW][HD + 4] (o
-    //      unnormalised, m, l) with agent-coherent stores, waits for them,
-    //      then arrives; the last to arrive merges all of them in segment
-    //      order (its own from registers) and puts the counter back to 0.
-    //      Nothing waits on another work-group.
-    constexpr int PS = HD + 4;
-    const size_t pblock = ((size_t)kvh * a.qblocks + blk) * a.nsp;
-    const __amdgpu_buffer_rsrc_t prs =
-        __builtin_amdgcn_make_buffer_rsrc(a.partials + pblock * S::RW * PS, 0, nsp * S::RW * PS * 4, 0x00020000);
-    int *counter = a.counters + ((size_t)kvh * a.qblocks + blk) * kCounterStrideP;
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const int r = (wave * NJ + j) * 16 + l16;
-        const int base = (sp * S::RW + r) * PS;
-#pragma unroll
-        for (int m = 0; m < S::MT; m++)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, st.o[m][j]), prs,
-                                                   (base + m * 16 + 4 * lg) * 4, 0, kCoherentP);
-        if (lg == 0) {
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(st.mrow[j]), prs, (base + HD) * 4, 0, kCoherentP);
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(lrow[j]), prs, (base + HD + 1) * 4, 0, kCoherentP);
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(0);   // this thread's partial is at the point of coherence
-    int *flag = reinterpret_cast<int *>(tile0);
-    __syncthreads();                 // every thread's partial; every wave done with the tile buffers
-    if (tid == 0) *flag = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nsp - 1;
-    __syncthreads();
-    if (!*flag) return;
-    if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const int r = (wave * NJ + j) * 16 + l16;
-        float M = -INFINITY, L = 0.0f;
-        v4f acc[S::MT];
-#pragma unroll
-        for (int m = 0; m < S::MT; m++) acc[m] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        for (int s2 = 0; s2 < nsp; s2++) {
-            const int base = (s2 * S::RW + r) * PS;
-            float ms, ls;
-            v4f os[S::MT];
-            if (s2 == sp) {
-                ms = st.mrow[j];
-                ls = lrow[j];
-#pragma unroll
-                for (int m = 0; m < S::MT; m++) os[m] = st.o[m][j];
-            } else {
-                ms = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(prs, (base + HD) * 4, 0, kCoherentP));
-                ls = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(prs, (base + HD + 1) * 4, 0, kCoherentP));
-#pragma unroll
-                for (int m = 0; m < S::MT; m++)
-                    os[m] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
-                                                        prs, (base + m * 16 + 4 * lg) * 4, 0, kCoherentP));
-            }
-            merge_part<S::MT>(M, L, acc, ms, ls, os);
-        }
-#pragma unroll
-        for (int m = 0; m < S::MT; m++) st.o[m][j] = acc[m];
-        lrow[j] = L;
-    }
-    store_rows<HD, G, NJ>(a, kvh, i0, wave, lane, st, lrow);
-}
-
-template <int HD, int G, int NJ>
-__global__ __launch_bounds__(kThreads, 2) void prefill_kernel(PrefillArgs a) {
-    using I = TileImg<HD>;
-    using S = PShape<HD, G, NJ>;
-    __shared__ __attribute__((aligned(16))) unsigned char tile0[I::BYTES];
-    __shared__ __attribute__((aligned(16))) unsigned char tile1[I::BYTES];
-    const int kvh = (int)blockIdx.x % a.n_kv;
-    const int item = (int)blockIdx.x / a.n_kv;
-    const int p = item / a.nsp, c = item % a.nsp;
-    // pair p: the later block bh, then the earlier bl (none for the middle block)
-    const int bh = a.qblocks - 1 - p, bl = p;
-    const int th = block_tiles(a.pos0, a.n, S::QB, bh);
-    const int tp = th + (bl < bh ? block_tiles(a.pos0, a.n, S::QB, bl) : 0);
-    const int C = (tp + a.nsp - 1) / a.nsp;             // tiles per chunk
-    const int c0 = c * C, c1 = min(tp, c0 + C);          // this chunk of the pair's sequence
-    if (c0 < min(c1, th))
-        prefill_segment<HD, G, NJ>(a, kvh, bh, c0, min(c1, th), c, (th + C - 1) / C, tile0, tile1);
-    if (c1 > max(c0, th)) {
-        __syncthreads();   // the LDS buffers are free again
-        prefill_segment<HD, G, NJ>(a, kvh, bl, max(c0, th) - th, c1 - th, c - th / C, (tp + C - 1) / C - th / C,
-                                   tile0, tile1);
-    }
-}
-
-// Whole query blocks: one work-group of 8 waves per (query block, kv head),
-// longest block first.  The two 4-wave halves cover the same 128 rows and
-// split the block's key tiles, half h taking tiles h, h + 2, h + 4, ...; they
-// step together (one barrier per pair of tiles, each half with its own two
-// LDS buffers, one tile ahead), then half 1 leaves its (o, m, l) in LDS and
-// half 0 merges the two in half order and stores the rows.  No partial leaves
-// the work-group and no work-group waits on another.
+// One work-group of 8 waves per (query block, run of its key tiles, kv head),
+// longest blocks first.  The two 4-wave halves cover the same 128 rows and
+// split the run, half h taking its tiles h, h + 2, h + 4, ...; they step
+// together (one barrier per pair of tiles, each half with its own two LDS
+// buffers, one tile ahead).  At the end each half hands one of its two row
+// tiles per wave to the other through LDS and merges its own with the one it
+// gets, in half order (NJ == 1: half 0 merges).
+//
+// A block covered by one run stores its rows.  With several, every work-group
+// writes its merged partial rows [RW][HD + 4] (o unnormalised, m, l) with
+// agent-coherent stores, waits for them, then arrives on the block's counter;
+// the last to arrive merges all of them in run order (its own from registers)
+// and puts the counter back to 0.  Nothing waits on another work-group.
 template <int HD, int G, int NJ>
 __global__ __launch_bounds__(2 * kThreads, 1) void prefill_block_kernel(PrefillArgs a) {
     using S = PShape<HD, G, NJ>;
     using I = TileImg<HD>;
     constexpr int MT = S::MT;
+    constexpr bool BOTH = NJ == 2;   // both halves finish a row tile per wave
     // tile buffers: half 0 uses 0, 1; half 1 uses 2, 3
     __shared__ __attribute__((aligned(16))) unsigned char tiles[4][I::BYTES];
-    static_assert(4 * 64 * (MT * NJ * 16 + NJ * 8) <= 4 * I::BYTES, "half 1's rows fit the tile buffers");
+    static_assert(2 * 4 * 64 * (MT * 16 + 8) <= 4 * I::BYTES, "the halves' row tiles fit the tile buffers");
     const int kvh = (int)blockIdx.x % a.n_kv;
-    const int blk = a.qblocks - 1 - (int)blockIdx.x / a.n_kv;
+    int blk = a.qblocks - 1, sp = (int)blockIdx.x / a.n_kv;
+    if (a.chunk == 0) {
+        blk -= sp;
+        sp = 0;
+    } else {
+        for (;; blk--) {
+            const int segs = block_runs(block_tiles(a.pos0, a.n, S::QB, blk), a.chunk);
+            if (sp < segs || blk == 0) break;
+            sp -= segs;
+        }
+    }
+    const int all = block_tiles(a.pos0, a.n, S::QB, blk);
+    const int segs = block_runs(all, a.chunk);
+    // runs of whole tile pairs, as even as they go
+    const int pairs = (all + 1) / 2;
+    const int kt0 = 2 * (pairs * sp / segs);
+    const int nt = min(all, 2 * (pairs * (sp + 1) / segs)) - kt0;
     const int tid = threadIdx.x;
     const int half = __builtin_amdgcn_readfirstlane(tid >> 8);
     const int htid = tid & (kThreads - 1);
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);   // wave within the half
     const int i0 = blk * S::QB;
-    const unsigned char *img = a.img + (size_t)kvh * a.n_tiles * I::BYTES;
-    const int nt = block_tiles(a.pos0, a.n, S::QB, blk);
+    const unsigned char *img = a.img + ((size_t)kvh * a.n_tiles + kt0) * I::BYTES;
     const int mine = (nt - half + 1) / 2;   // tiles of this half
     const int steps = (nt + 1) / 2;         // half 0 has the most
 
@@ -1050,48 +922,116 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_block_kernel(PrefillA
         asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
         __syncthreads();
         if (s + 1 < mine) fetch_tile<HD>(img, 2 * (s + 1) + half, buf(s + 1), htid, wave);
-        if (s < mine) tile_update<HD, G, NJ>(a, buf(s), 2 * s + half, i0, lane, q, st);
+        if (s < mine) tile_update<HD, G, NJ>(a, buf(s), kt0 + 2 * s + half, i0, lane, q, st);
     }
 
     float lrow[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) lrow[j] = xrow_sum(st.lsum[j]);
-    // half 1's rows, lane by lane (the waves of both halves hold the same
-    // rows and columns in the same lanes), into the free tile buffers
-    v4f *ob = reinterpret_cast<v4f *>(&tiles[0][0]);              // [wave][MT][NJ][64]
-    float *mb = reinterpret_cast<float *>(ob + 4 * MT * NJ * 64);  // [wave][NJ][64] x (m, l)
+    // row tile j of a half is finished by half j (BOTH) or half 0; the other
+    // half leaves it in the free tile buffers lane by lane (the waves of both
+    // halves hold the same rows and columns in the same lanes)
+    v4f *ob = reinterpret_cast<v4f *>(&tiles[0][0]);               // [from half][wave][MT][64]
+    float *mb = reinterpret_cast<float *>(ob + 2 * 4 * MT * 64);   // [from half][wave][64] x (m, l)
     __syncthreads();   // every wave is done with the tile buffers
-    if (half == 1) {
+    v4f acc[MT];
+    float M = -INFINITY, L = 0.0f;
+    {
+        v4f own[MT], os[MT];
+        float om, ol;
+        const int at = half * 4 + wave, from = (1 - half) * 4 + wave;
+        if (BOTH || half == 1) {
 #pragma unroll
-        for (int m = 0; m < MT; m++)
-#pragma unroll
-            for (int j = 0; j < NJ; j++) ob[((wave * MT + m) * NJ + j) * 64 + lane] = st.o[m][j];
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            mb[((wave * NJ + j) * 64 + lane) * 2] = st.mrow[j];
-            mb[((wave * NJ + j) * 64 + lane) * 2 + 1] = lrow[j];
+            for (int m = 0; m < MT; m++)
+                ob[(at * MT + m) * 64 + lane] = BOTH && half == 0 ? st.o[m][NJ - 1] : st.o[m][0];
+            mb[(at * 64 + lane) * 2] = BOTH && half == 0 ? st.mrow[NJ - 1] : st.mrow[0];
+            mb[(at * 64 + lane) * 2 + 1] = BOTH && half == 0 ? lrow[NJ - 1] : lrow[0];
         }
-    }
-    __syncthreads();
-    if (half == 1) return;
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        float M = -INFINITY, L = 0.0f;
-        v4f acc[MT], os[MT];
+        const bool last = BOTH && half == 1;   // this half keeps its last row tile
 #pragma unroll
         for (int m = 0; m < MT; m++) {
             acc[m] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-            os[m] = st.o[m][j];
+            own[m] = last ? st.o[m][NJ - 1] : st.o[m][0];
         }
-        merge_part<MT>(M, L, acc, st.mrow[j], lrow[j], os);
+        const float mo = last ? st.mrow[NJ - 1] : st.mrow[0], lo = last ? lrow[NJ - 1] : lrow[0];
+        __syncthreads();
+        if (!BOTH && half == 1 && segs == 1) return;
+        if (BOTH || half == 0) {
 #pragma unroll
-        for (int m = 0; m < MT; m++) os[m] = ob[((wave * MT + m) * NJ + j) * 64 + lane];
-        merge_part<MT>(M, L, acc, mb[((wave * NJ + j) * 64 + lane) * 2], mb[((wave * NJ + j) * 64 + lane) * 2 + 1], os);
-#pragma unroll
-        for (int m = 0; m < MT; m++) st.o[m][j] = acc[m];
-        lrow[j] = L;
+            for (int m = 0; m < MT; m++) os[m] = ob[(from * MT + m) * 64 + lane];
+            om = mb[(from * 64 + lane) * 2];
+            ol = mb[(from * 64 + lane) * 2 + 1];
+            if (half == 0) {
+                merge_part<MT>(M, L, acc, mo, lo, own);
+                merge_part<MT>(M, L, acc, om, ol, os);
+            } else {
+                merge_part<MT>(M, L, acc, om, ol, os);
+                merge_part<MT>(M, L, acc, mo, lo, own);
+            }
+        }
     }
-    store_rows<HD, G, NJ>(a, kvh, i0, wave, lane, st, lrow);
+    const bool mine_rows = BOTH || half == 0;
+    const int tile = wave * NJ + (BOTH ? half : 0);   // the row tile this wave finishes
+    if (segs == 1) {
+        store_rows<HD, G, NJ>(a, kvh, i0, tile, lane, acc, L);
+        return;
+    }
+
+    const int l16 = lane & 15, lg = lane >> 4;
+    constexpr int PS = HD + 4;
+    const size_t pblock = ((size_t)kvh * a.qblocks + blk) * a.nsp;
+    const __amdgpu_buffer_rsrc_t prs =
+        __builtin_amdgcn_make_buffer_rsrc(a.partials + pblock * S::RW * PS, 0, segs * S::RW * PS * 4, 0x00020000);
+    int *counter = a.counters + ((size_t)kvh * a.qblocks + blk) * kCounterStrideP;
+    const int r = tile * 16 + l16;
+    if (mine_rows) {
+        const int base = (sp * S::RW + r) * PS;
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[m]), prs, (base + m * 16 + 4 * lg) * 4,
+                                                   0, kCoherentP);
+        if (lg == 0) {
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(M), prs, (base + HD) * 4, 0, kCoherentP);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(L), prs, (base + HD + 1) * 4, 0, kCoherentP);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0);   // this thread's partial is at the point of coherence
+    int *flag = reinterpret_cast<int *>(&tiles[0][0]);
+    __syncthreads();                 // every thread's partial; every wave done with the exchanged rows
+    if (tid == 0) *flag = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == segs - 1;
+    __syncthreads();
+    if (!*flag || !mine_rows) return;
+    if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+    // the runs' partials, the next one's loads in flight while one is merged
+    float M2 = -INFINITY, L2 = 0.0f;
+    v4f acc2[MT], os[2][MT];
+    float ms[2], ls[2];
+#pragma unroll
+    for (int m = 0; m < MT; m++) acc2[m] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    auto load = [&](int s2, v4f (&o)[MT], float &m1, float &l1) {
+        const int base = (s2 * S::RW + r) * PS;
+        m1 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(prs, (base + HD) * 4, 0, kCoherentP));
+        l1 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(prs, (base + HD + 1) * 4, 0, kCoherentP));
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+            o[m] = __builtin_bit_cast(
+                v4f, __builtin_amdgcn_raw_buffer_load_b128(prs, (base + m * 16 + 4 * lg) * 4, 0, kCoherentP));
+    };
+    auto fold = [&](int s2, const v4f (&o)[MT], float m1, float l1) {
+        if (s2 == sp)
+            merge_part<MT>(M2, L2, acc2, M, L, acc);
+        else
+            merge_part<MT>(M2, L2, acc2, m1, l1, o);
+    };
+    load(0, os[0], ms[0], ls[0]);
+    for (int s2 = 0; s2 < segs; s2 += 2) {
+        if (s2 + 1 < segs) load(s2 + 1, os[1], ms[1], ls[1]);
+        fold(s2, os[0], ms[0], ls[0]);
+        if (s2 + 2 < segs) load(s2 + 2, os[0], ms[0], ls[0]);
+        if (s2 + 1 < segs) fold(s2 + 1, os[1], ms[1], ls[1]);
+    }
+    store_rows<HD, G, NJ>(a, kvh, i0, tile, lane, acc2, L2);
 }
 
 // Rows per work-group: 128 (two row tiles per wave) by default;
@@ -1109,56 +1049,60 @@ int prefill_rows(int g) {
 int prefill_qb(int g) { return 64 * (prefill_rows(g) == 128 ? 2 : 1) / g; }
 
 // With at least two query blocks per CU, every (query block, kv head) is one
-// work-group of prefill_block_kernel (no partials): dealt longest first, the
-// blocks pair up on the CUs by themselves.  With fewer, query blocks are
-// paired last with first and cut into nsp chunks, the count that minimises
-// the time of the item waves (items of ceil(tp/nsp) tiles each,
-// kItemOverheadTiles extra, resident work-groups at once per wave), run by
-// prefill_kernel with split partials.
+// work-group: dealt longest first, the blocks pair up on the CUs by
+// themselves.  With fewer, blocks may be cut into runs of `chunk` key tiles,
+// the length that minimises the modelled time: one work-group's (steps, fixed
+// cost, the merge of all runs by the last) while the launch is one round of
+// the CUs, else the CUs' share of all work plus half a work-group's.
+// Measured (us with 1, 2, 3, 4 and 8 runs of the longest block, 32 / 8 heads
+// of 128): 333 tokens after 1,000: 56.4 / 45.7 / 57.3 / 56.2 / 56.5; 100 after
+// 8,000: 255 / 149 / 112 / 95 / 74; 300 after none: 24.3 / 28.6 / 28.7 / - / -;
+// 1,024 after 1,024: 79.3 / 91 / 107 / 128 / 190; 8 / 2 heads of 64, 2,048
+// after none: 50 / 35 / 32 / 38 / 42.  The plan takes 2, 8, 1, 1 and 3.
 constexpr int kCUs = 256;                // compute units of an MI355X
-// TQ_HIP_PREFILL_WHOLE=1|0 forces the whole-block kernel or the paired split
-// one (tests of both at any size); read on every call.  -1: the plan decides.
+// TQ_HIP_PREFILL_WHOLE=1 keeps every block one run, =0 cuts every block into
+// as many runs as the plan may (tests of both at any size); read on every
+// call.  -1: the plan decides.
 int prefill_whole_env() {
     const char *s = getenv("TQ_HIP_PREFILL_WHOLE");
     return (s && *s) ? (s[0] == '1' ? 1 : 0) : -1;
 }
 struct PrefillPlan {
-    int qblocks, nsp, rows, items;
-    bool whole;                          // prefill_block_kernel
+    int qblocks, chunk, nsp, rows, items;
 };
 PrefillPlan plan_prefill(int hd, int g, int n_kv_heads, int pos0, int n) {
     PrefillPlan p;
     const int qb = prefill_qb(g);
     p.rows = 64 * (prefill_rows(g) == 128 ? 2 : 1);
     p.qblocks = (n + qb - 1) / qb;
-    const int forced = prefill_whole_env();
-    p.whole = forced >= 0 ? forced == 1 : (long)p.qblocks * n_kv_heads >= 2L * kCUs;
-    if (p.whole) {
-        p.nsp = 1;
-        p.items = p.qblocks;
-        return p;
-    }
-    const int pairs = (p.qblocks + 1) / 2;
-    int tp_max = 0;
-    for (int q = 0; q < pairs; q++) {
-        const int bh = p.qblocks - 1 - q;
-        const int tp = block_tiles(pos0, n, qb, bh) + (q < bh ? block_tiles(pos0, n, qb, q) : 0);
-        tp_max = std::max(tp_max, tp);
-    }
-    const long slots = 256L * (hd == 128 ? 2 : 4);   // resident work-groups: 2 or 4 per CU
-    long best = -1;
+    p.chunk = 0;
     p.nsp = 1;
-    for (int k = 1; k <= kMaxSplitsP; k++) {
-        const int C = (tp_max + k - 1) / k;
-        if (k > 1 && C < 4) break;
-        const long waves = ((long)pairs * k * n_kv_heads + slots - 1) / slots;
-        const long cost = waves * (C + kItemOverheadTiles);
-        if (best < 0 || cost < best) {
+    p.items = p.qblocks;
+    const int forced = prefill_whole_env();
+    if (forced == 1 || (forced < 0 && (long)p.qblocks * n_kv_heads >= 2L * kCUs)) return p;
+    const int most = block_tiles(pos0, n, qb, p.qblocks - 1);   // of the last, longest block
+    const double unit = hd == 128 ? 1.0 : 1.5;                  // the fixed costs in steps, which are shorter at 64
+    double best = 0.0;
+    for (int k = 1; k <= kMaxRuns && (k == 1 || (most + 1) / 2 >= k); k++) {
+        const int chunk = (((most + k - 1) / k) + 1) & ~1;
+        long items = 0, tiles = 0;
+        for (int b = 0; b < p.qblocks; b++) {
+            const int nt = block_tiles(pos0, n, qb, b);
+            items += block_runs(nt, chunk);
+            tiles += nt;
+        }
+        const int runs = block_runs(most, chunk);
+        const double item = unit * (kItemCost + (runs > 1 ? kRunCost : 0.0));
+        const double one = 0.5 * chunk + item + (runs > 1 ? unit * kMergeCost * runs : 0.0);
+        const double work = n_kv_heads * (0.5 * tiles + items * item) / kCUs;
+        const double cost = items * n_kv_heads <= kCUs ? one : std::max(one, work + 0.5 * one);
+        if (forced == 0 || k == 1 || cost < best) {
             best = cost;
-            p.nsp = k;
+            p.chunk = k == 1 ? 0 : chunk;
+            p.nsp = runs;
+            p.items = (int)items;
         }
     }
-    p.items = pairs * p.nsp;
     return p;
 }
 
@@ -1172,7 +1116,7 @@ size_t qimg_offset(int head_dim, int n_kv_heads, int kend) {
 
 // The staging launch (key tiles and q blocks), then the attention.
 template <int HD, int G, int NJ>
-hipError_t launch_hd_g(const TqPrefillArgs &t, const PrefillArgs &a, bool whole, hipStream_t s) {
+hipError_t launch_hd_g(const TqPrefillArgs &t, const PrefillArgs &a, int items, hipStream_t s) {
     StageArgs st;
     st.view = t.view;
     st.seq = t.seq;
@@ -1198,24 +1142,18 @@ hipError_t launch_hd_g(const TqPrefillArgs &t, const PrefillArgs &a, bool whole,
                        0, s, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (whole) {
-        hipLaunchKernelGGL((prefill_block_kernel<HD, G, NJ>), dim3(a.qblocks * t.n_kv_heads), dim3(2 * kThreads), 0,
-                           s, a);
-    } else {
-        const int items = (a.qblocks + 1) / 2 * a.nsp;
-        hipLaunchKernelGGL((prefill_kernel<HD, G, NJ>), dim3(items * t.n_kv_heads), dim3(kThreads), 0, s, a);
-    }
+    hipLaunchKernelGGL((prefill_block_kernel<HD, G, NJ>), dim3(items * t.n_kv_heads), dim3(2 * kThreads), 0, s, a);
     return hipGetLastError();
 }
 
 template <int HD>
-hipError_t launch_hd(const TqPrefillArgs &t, const PrefillArgs &a, int g, bool whole, hipStream_t s) {
+hipError_t launch_hd(const TqPrefillArgs &t, const PrefillArgs &a, int g, int items, hipStream_t s) {
     const bool wide = prefill_rows(g) == 128;
     switch (g) {
-        case 1: return wide ? launch_hd_g<HD, 1, 2>(t, a, whole, s) : launch_hd_g<HD, 1, 1>(t, a, whole, s);
-        case 2: return wide ? launch_hd_g<HD, 2, 2>(t, a, whole, s) : launch_hd_g<HD, 2, 1>(t, a, whole, s);
-        case 4: return wide ? launch_hd_g<HD, 4, 2>(t, a, whole, s) : launch_hd_g<HD, 4, 1>(t, a, whole, s);
-        case 8: return launch_hd_g<HD, 8, 2>(t, a, whole, s);
+        case 1: return wide ? launch_hd_g<HD, 1, 2>(t, a, items, s) : launch_hd_g<HD, 1, 1>(t, a, items, s);
+        case 2: return wide ? launch_hd_g<HD, 2, 2>(t, a, items, s) : launch_hd_g<HD, 2, 1>(t, a, items, s);
+        case 4: return wide ? launch_hd_g<HD, 4, 2>(t, a, items, s) : launch_hd_g<HD, 4, 1>(t, a, items, s);
+        case 8: return launch_hd_g<HD, 8, 2>(t, a, items, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1231,7 +1169,7 @@ bool tq_prefill_mfma_supported(int head_dim, int group, int kend) {
 void tq_prefill_scratch(int head_dim, int group, int n_kv_heads, int pos0, int n, size_t *partial_bytes,
                         size_t *counter_ints) {
     const PrefillPlan p = plan_prefill(head_dim, group, n_kv_heads, pos0, n);
-    if (p.whole || p.nsp == 1) {
+    if (p.nsp == 1) {
         *partial_bytes = 0;
         *counter_ints = 0;
         return;
@@ -1261,10 +1199,11 @@ hipError_t tq_launch_prefill(const TqPrefillArgs &t, hipStream_t s) {
     a.qimg = t.img + qimg_offset(t.head_dim, t.n_kv_heads, t.pos0 + t.n);
     const PrefillPlan p = plan_prefill(t.head_dim, g, t.n_kv_heads, t.pos0, t.n);
     a.qblocks = p.qblocks;
+    a.chunk = p.chunk;
     a.nsp = p.nsp;
     a.n_kv = t.n_kv_heads;
     a.partials = t.partials;
     a.counters = t.counters;
     if (p.nsp > 1 && (!t.partials || !t.counters)) return hipErrorInvalidValue;
-    return t.head_dim == 64 ? launch_hd<64>(t, a, g, p.whole, s) : launch_hd<128>(t, a, g, p.whole, s);
+    return t.head_dim == 64 ? launch_hd<64>(t, a, g, p.items, s) : launch_hd<128>(t, a, g, p.items, s);
 }

@@ -558,6 +558,33 @@ def test_prefill_both_plans(nat, oracle, shape, whole, monkeypatch):
     check_prefill(nat, oracle, shape)
 
 
+@pytest.mark.parametrize("pos0,n", [(0, 33), (0, 95), (31, 64), (97, 40), (480, 33), (700, 130)])
+@pytest.mark.parametrize("nq,nkv,hd", [(32, 8, 128), (8, 2, 64), (4, 4, 64), (8, 1, 128)])
+def test_prefill_runs(nat, oracle, nq, nkv, hd, pos0, n, monkeypatch):
+    """Query blocks cut into as many runs of key tiles as the plan allows: runs
+    of one tile (a half without any), runs that rows near the diagonal see no
+    key of, blocks with fewer runs than others; the same against one run per
+    block (only the order of the fp32 sums differs: a row's share of each of
+    the T keys is within T 2^-22 of its size, weights and values are O(1))."""
+    T = pos0 + n
+    monkeypatch.setenv("TQ_HIP_PREFILL_WHOLE", "0")
+    check_prefill(nat, oracle, (nq, nkv, hd, T, 1e4, pos0, n))
+    q, k, v = (normal(n * h * hd, 30 + i) for i, h in enumerate((nq, nkv, nkv)))
+    pre = [oracle.quantize_row_q8(normal(nkv * T * hd, 40 + i)).reshape(nkv, T, hd // QK) for i in range(2)]
+    outs = []
+    for whole in ("0", "1", "0"):
+        monkeypatch.setenv("TQ_HIP_PREFILL_WHOLE", whole)
+        kv = nat.PagedKV.single(nq, nkv, hd, T)
+        kv.write(0, 0, *pre)
+        rc, out = kv.prefill(0, pos0, n, q, k, v)
+        assert rc == 0
+        outs.append(out)
+        kv.close()
+    assert outs[0].tobytes() == outs[2].tobytes()
+    err = np.abs(outs[0].astype(np.float64) - outs[1])
+    assert err.max() <= T * 2.0 ** -22 * np.abs(outs[1]).max(), err.max()
+
+
 def check_prefill(nat, oracle, shape):
     nq, nkv, hd, T, theta, pos0, n = shape
     nb = hd // QK
