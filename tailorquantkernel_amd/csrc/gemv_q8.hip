@@ -214,26 +214,22 @@ __device__ __forceinline__ void dma4(const void *src, unsigned char *dst) {
 }
 
 // The same copies from a uniform base plus a 32-bit lane offset (the saddr
-// form): no per-lane 64-bit address arithmetic.  base and dst are uniform.
-__device__ __forceinline__ void dma16s(const unsigned char *base, uint32_t off, unsigned char *dst) {
-    const uint32_t lds = (uint32_t)(uintptr_t)(lds_u8 *)dst;
-    uint32_t saved;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\t"
-        "global_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(off), "s"(base), "s"(lds)
-        : "memory");
+// form) to LDS byte address lds + IMM: no per-lane 64-bit address arithmetic,
+// and two scalar instructions with the copy (M0 is left changed; nothing else
+// in these kernels uses it).  base and lds are uniform.
+template <int IMM>
+__device__ __forceinline__ void dma16s(const unsigned char *base, uint32_t off, uint32_t lds) {
+    asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(off), "s"(base), "s"(lds), "n"(IMM)
+                 : "m0", "scc", "memory");
 }
-__device__ __forceinline__ void dma4s(const unsigned char *base, uint32_t off, unsigned char *dst) {
-    const uint32_t lds = (uint32_t)(uintptr_t)(lds_u8 *)dst;
-    uint32_t saved;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\t"
-        "global_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(off), "s"(base), "s"(lds)
-        : "memory");
+template <int IMM>
+__device__ __forceinline__ void dma4s(const unsigned char *base, uint32_t off, uint32_t lds) {
+    asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dword %0, %1"
+                 :
+                 : "v"(off), "s"(base), "s"(lds), "n"(IMM)
+                 : "m0", "scc", "memory");
 }
 
 // `bytes` (a multiple of 4) from src into LDS at dst, all by DMA: whole
@@ -484,9 +480,10 @@ static_assert(kGemmA / 16 % kGemmThreads == 0 && kGemmKB * kGemmRows == kGemmThr
               kGemmBWords % kGemmThreads == 0, "whole copy rounds per stage");
 
 // Slot of a stage's block (0..3) in its row's 64 bytes of codes (its own
-// inverse): any 8 consecutive rows then hold a block in 8 different 16-byte
-// bank groups.
-__device__ __forceinline__ int gemm_slot(int blk, int row) { return blk ^ ((row >> 1) & 3); }
+// inverse): any 16 consecutive rows then hold a block in 16 different 16-byte
+// bank groups (a 16-byte read of 64 lanes takes 4 cycles; 8 when two of 16
+// rows share one, 16 without the permutation).
+__device__ __forceinline__ int gemm_slot(int blk, int row) { return blk ^ ((row >> 2) & 3); }
 
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -608,49 +605,81 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         }
     }
 
-    // the same copies from uniform bases (whole stages only)
-    auto issue_uni = [&](int st, unsigned char *buf) {
+    // The same copies from uniform bases (whole stages only): each copy of a
+    // stage has its own base, which moves on by a fixed step from stage to
+    // stage (the weight codes jump at the end of a 64-block group), so a
+    // copy costs three or four scalar instructions.  (Recomputing the bases
+    // from the stage number took about 100 per stage and wave, issued in order
+    // in front of its products: attention layer over 2,048 rows 354 us, now
+    // 351; Q4 MLP over 100 rows 104.3, now 103.4.)
+    const unsigned char *pw0 = nullptr, *pw1 = nullptr, *pd = nullptr, *px[2] = {nullptr, nullptr}, *pxd = nullptr;
+    int in_group = 0;   // blocks of the current group already copied
+    int group_left = 0; // blocks of the row from the current group on
+    size_t xstep = 0;
+    auto start_uni = [&](int st) {
         const int b0 = st * kGemmKB;
-        const int g = b0 / kGroupBlocks, i0 = b0 - g * kGroupBlocks;
-        const int n = nb - g * kGroupBlocks < kGroupBlocks ? nb - g * kGroupBlocks : kGroupBlocks;
+        const int g = b0 / kGroupBlocks;
+        in_group = b0 - g * kGroupBlocks;
+        group_left = nb - g * kGroupBlocks;
+        const int n = group_left < kGroupBlocks ? group_left : kGroupBlocks;
         if (Q4) {
-            dma16s(useg + 16 * b0, vrow, buf + 16 * 64 * wave);
+            pw0 = useg + 16 * b0;
         } else {
-#pragma unroll
-            for (int half = 0; half < 2; half++)
-                dma16s(useg + g * kGroupBytes + 16 * (i0 + half * n), vrow, buf + 16 * (64 * wave + kGemmThreads * half));
+            pw0 = useg + g * kGroupBytes + 16 * in_group;
+            pw1 = pw0 + 16 * n;
         }
-        if (wave < 2) dma16s(uwd + uscale + 4 * b0, vdrow, buf + kGemmA + 16 * 64 * wave);
+        pd = uwd + uscale + 4 * b0;
         if constexpr (XS) {
             // codes: chunk c -> (block c / 256, half (c / 128) & 1, token c % 128),
-            // the same [block][half][row] 16-byte layout as the weights, one
-            // contiguous KiB per wave; scales: dword c -> (block c / 128, token c % 128)
+            // the wave's two: half (wave / 2) & 1 of blocks wave / 4 and 2 + wave / 4;
+            // scales: dword c -> (block c / 128, token c % 128), block wave / 2
             const size_t n16 = 16 * (size_t)a.n_tok;
-#pragma unroll
-            for (int j = 0; j < kGemmA / 16 / kGemmThreads; j++) {
-                const int c = 64 * wave + kGemmThreads * j;
-                const int blk = c >> 8, half = (c >> 7) & 1;
-                dma16s(a.xq + (size_t)(2 * (b0 + blk) + half) * n16 + 16 * tok0, vb[0] - 16u * (uint32_t)tok0,
-                       buf + kGemmA + kGemmWD + 16 * c);
-            }
-            dma4s(a.xq + (size_t)a.n_tok * cols + 4 * ((size_t)(b0 + (wave >> 1)) * a.n_tok + tok0),
-                  vb[1] - 4u * (uint32_t)tok0, buf + kGemmA + kGemmWD + kGemmXsCodes + sdst);
+            xstep = 2 * kGemmKB * n16;
+            px[0] = a.xq + (size_t)(2 * (b0 + (wave >> 2)) + ((wave >> 1) & 1)) * n16;
+            px[1] = px[0] + 4 * n16;
+            pxd = a.xq + (size_t)a.n_tok * cols + 4 * (size_t)(b0 + (wave >> 1)) * a.n_tok;
         } else {
-#pragma unroll
-            for (int j = 0; j < kGemmBRounds; j++) {
-                const int c = 64 * wave + kGemmThreads * j;
-                if (c < kGemmBChunks)
-                    dma16s(a.xq + (size_t)b0 * kBlockBytes, vb[j], buf + kGemmA + kGemmWD + 16 * c);
+            px[0] = a.xq + (size_t)b0 * kBlockBytes;
+        }
+    };
+    auto issue_uni = [&](uint32_t buf) {
+        const uint32_t at = buf + 16 * 64 * wave;   // the wave's KiB of a round of copies
+        dma16s<0>(pw0, vrow, at);
+        if (!Q4) dma16s<16 * kGemmThreads>(pw1, vrow, at);
+        if (wave < 2) dma16s<kGemmA>(pd, vdrow, at);
+        if constexpr (XS) {
+            dma16s<kGemmA + kGemmWD>(px[0], vb[0], at);
+            dma16s<kGemmA + kGemmWD + 16 * kGemmThreads>(px[1], vb[0], at);
+            dma4s<kGemmA + kGemmWD + kGemmXsCodes>(pxd, vb[1], buf + sdst);
+            px[0] += xstep;
+            px[1] += xstep;
+            pxd += xstep / 8;
+        } else {
+            dma16s<kGemmA + kGemmWD>(px[0], vb[0], at);
+            dma16s<kGemmA + kGemmWD + 16 * kGemmThreads>(px[0], vb[1], at);
+            static_assert(kGemmBRounds == 3 && kGemmBChunks - 2 * kGemmThreads == 128, "the third round is two waves'");
+            if (wave < 2) dma16s<kGemmA + kGemmWD + 32 * kGemmThreads>(px[0], vb[2], at);
+            px[0] += kGemmKB * kBlockBytes;
+        }
+        pd += 4 * kGemmKB;
+        if (Q4) {
+            pw0 += 16 * kGemmKB;
+        } else {
+            pw0 += 16 * kGemmKB;
+            pw1 += 16 * kGemmKB;
+            in_group += kGemmKB;
+            if (in_group == kGroupBlocks) {
+                // the next group starts after this one's last halves
+                pw0 += 16 * kGroupBlocks;
+                in_group = 0;
+                group_left -= kGroupBlocks;
+                pw1 = pw0 + 16 * (group_left < kGroupBlocks ? group_left : kGroupBlocks);
             }
         }
     };
 
     // kGemmCopies direct-to-LDS copies per thread per stage, nothing else
     auto issue = [&](int st, unsigned char *buf) {
-        if constexpr (uni) {
-            issue_uni(st, buf);
-            return;
-        }
         const int b0 = st * kGemmKB;
         const int bw = b0 + my_blk < nb ? b0 + my_blk : nb - 1;
         if (Q4) {
@@ -687,12 +716,23 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
 
     // Two buffers (73.7 KB, so two work-groups share a CU): stage st+1 is
     // copied while stage st is multiplied.
-    issue(st_begin, smem);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_u8 *)smem;
+    if constexpr (uni) {
+        start_uni(st_begin);
+        issue_uni(lds0);
+    } else {
+        issue(st_begin, smem);
+    }
     for (int st = st_begin; st < st_end; st++) {
         unsigned char *buf = smem + ((st - st_begin) & 1) * kGemmStage;
         wait_vm<0>();      // this wave's copies of stage st have landed
         __syncthreads();   // stage st is in LDS everywhere; stage st-1's buffer is free
-        if (st + 1 < st_end) issue(st + 1, smem + ((st + 1 - st_begin) & 1) * kGemmStage);
+        if (st + 1 < st_end) {
+            if constexpr (uni)
+                issue_uni(lds0 + (((st + 1 - st_begin) & 1) ? kGemmStage : 0));
+            else
+                issue(st + 1, smem + ((st + 1 - st_begin) & 1) * kGemmStage);
+        }
         const unsigned char *A = buf, *WD = buf + kGemmA, *B = buf + kGemmA + kGemmWD;
         // the row's four scales (times 1/16 for the Q4 codes, which come as 16 x code)
         float4 wd4 = *reinterpret_cast<const float4 *>(WD + (wr + l32) * 16);
