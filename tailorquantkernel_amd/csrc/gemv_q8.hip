@@ -54,6 +54,8 @@
 
 #include <stdlib.h>
 
+#include <algorithm>
+
 namespace {
 
 using namespace tq;
@@ -171,7 +173,10 @@ struct GemvArgs {
     unsigned char *hq;        // GEMM over the MLP's gate (segment 0) and up (segment 1)
                               // matrices: each tile pairs 64 rows of both, and the
                               // epilogue writes silu_mul + quantize_row_q8 of the
-                              // hidden rows in the split layout here instead of y
+                              // hidden rows in the split layout here instead of y;
+                              // with K splits the reduce launch does so beside y,
+                              // in the split layout or (hq_xs false) as block_q8 rows
+    bool hq_xs;
 };
 
 typedef __attribute__((address_space(3))) unsigned char lds_u8;
@@ -417,8 +422,11 @@ size_t lds_bytes(int t, int nb, bool xf) {
 
 // ---------------------------------------------------------------------------
 // Many tokens: int8 MFMA GEMM.  A work-group of 8 waves computes a 128-row x
-// 128-token tile; wave w owns rows 32(w%4)..+31 of tokens 64(w/4)..+63, two
-// 32 x 32 tiles.  The K dimension goes 4 blocks (128 codes) per stage through
+// 128-token tile (TT = 128), or 64 tokens where a launch has no more; wave w
+// owns rows 32(w%4)..+31 of tokens 64(w/4)..+63 (32(w/4)..+31), two 32 x 32
+// tiles (one).  The smaller tile halves the products and the token copies
+// per weight byte: 28,672 x 4,096 over 64 tokens 49 us against 67 with 128
+// tokens' tile.  The K dimension goes 4 blocks (128 codes) per stage through
 // two LDS buffers filled by direct-to-LDS copies, one stage ahead of the one
 // being multiplied; at 74.8 KB and 128 registers two work-groups share a CU,
 // four waves per SIMD.
@@ -449,35 +457,38 @@ size_t lds_bytes(int t, int nb, bool xf) {
 // (work-group w: XCD w % 8, row tile 8 (w/8 / n_tt) + w % 8) and the tile's
 // 128 weight rows are read from HBM once into that XCD's L2.
 //
-// LDS per stage (37,376 B):
+// LDS per stage (37,376 B; 28,160 with 64 tokens):
 //   A   [2 halves][128 rows][4 slots][16 B]   weight codes (Q4: one nibble run
 //       instead of two halves), block b of row r in slot gemm_slot(b, r)
 //   WD  [128 rows][4 blocks] fp32             weight scales
 //   B   [128 tokens][4 blocks x 36 B]         the tokens' block_q8, as stored:
 //       with 16-byte aligned rows and a block count that is a multiple of 4,
-//       a token's 144 bytes are nine 16-byte copies (three rounds of 512, the
-//       last round's surplus lanes, whole waves, issue none); otherwise 36
-//       dword copies per token.  Or, from the split layout, codes
+//       a token's 144 bytes are nine 16-byte copies (rounds of 512, the last
+//       one's surplus lanes, whole waves, issue none); otherwise 36 dword
+//       copies per token.  Or, from the split layout, codes
 //       [4 blocks][2 halves][128 tokens][16 B], then scales
 //       [4 blocks][128 + 32 tokens] fp32 (two blocks' rows in other banks).
 constexpr int kGemmThreads = 512;
-constexpr int kGemmRows = 128, kGemmToks = 128, kGemmKB = 4, kGemmBufs = 2;
+constexpr int kGemmRows = 128, kGemmKB = 4, kGemmBufs = 2;
 constexpr int kGemmA = kGemmKB * 2 * kGemmRows * 16;            // 16,384
 constexpr int kGemmWD = kGemmKB * kGemmRows * 4;                // 2,048
-constexpr int kGemmScaleRow = kGemmToks + 32;                   // floats between two blocks' token scales
 constexpr int kGemmBRow = kGemmKB * kBlockBytes;                // 144 bytes per token
-constexpr int kGemmBRows = kGemmToks * kGemmBRow;               // 18,432
-constexpr int kGemmBChunks = kGemmBRows / 16;                   // 1,152 16-byte copies
-constexpr int kGemmBRounds = (kGemmBChunks + kGemmThreads - 1) / kGemmThreads;   // 3
-constexpr int kGemmBWords = kGemmBRows / 4;                     // 4,608 dword copies
-constexpr int kGemmXsCodes = kGemmKB * kQK * kGemmToks;         // 16,384: split-layout codes, then scales
-constexpr int kGemmB = kGemmXsCodes + kGemmKB * kGemmScaleRow * 4;   // 18,944
-constexpr int kGemmStage = kGemmA + kGemmWD + kGemmB;           // 37,376
-static_assert(kGemmBRows <= kGemmB && kGemmStage % 16 == 0 && kGemmToks == kGemmRows, "stage layout");
-static_assert(kGemmBChunks % 64 == 0 && (kGemmBRounds - 1) * kGemmThreads < kGemmBChunks,
-              "the last B round's copies past the tile are whole waves");
-static_assert(kGemmA / 16 % kGemmThreads == 0 && kGemmKB * kGemmRows == kGemmThreads &&
-              kGemmBWords % kGemmThreads == 0, "whole copy rounds per stage");
+static_assert(kGemmA / 16 == 2 * kGemmThreads && kGemmKB * kGemmRows == kGemmThreads, "whole weight copy rounds per stage");
+
+// Sizes that depend on a tile's tokens (128 or 64).
+template <int TT>
+struct GemmTile {
+    static constexpr int T2 = TT / 64;                              // 32-token tiles per wave
+    static constexpr int ROWS = TT * kGemmBRow;                     // block_q8 rows: 18,432 or 9,216
+    static constexpr int CHUNKS = ROWS / 16;                        // 16-byte copies
+    static constexpr int ROUNDS = (CHUNKS + kGemmThreads - 1) / kGemmThreads;
+    static constexpr int WORDS = ROWS / 4;                          // dword copies
+    static constexpr int SROW = TT + 32;                            // floats between two blocks' token scales
+    static constexpr int CODES = kGemmKB * kQK * TT;                // split-layout codes, then scales
+    static constexpr int B = CODES + kGemmKB * SROW * 4;            // 18,944 or 9,728
+    static constexpr int STAGE = kGemmA + kGemmWD + B;              // 37,376 or 28,160
+    static_assert(ROWS <= B && STAGE % 16 == 0 && CHUNKS % 64 == 0 && WORDS % 64 == 0, "stage layout, whole waves");
+};
 
 // Slot of a stage's block (0..3) in its row's 64 bytes of codes (its own
 // inverse): any 16 consecutive rows then hold a block in 16 different 16-byte
@@ -486,6 +497,7 @@ static_assert(kGemmA / 16 % kGemmThreads == 0 && kGemmKB * kGemmRows == kGemmThr
 __device__ __forceinline__ int gemm_slot(int blk, int row) { return blk ^ ((row >> 2) & 3); }
 
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v32f __attribute__((ext_vector_type(32)));
 
@@ -494,17 +506,19 @@ typedef float v32f __attribute__((ext_vector_type(32)));
 // copy per thread instead of two); each lane turns its 8 bytes into 16 x its
 // 8 codes (low nibbles for k < 16, high for k >= 16), and the int32 products
 // are shifted back by 4 before scaling.
-template <bool BX4, bool Q4, bool UNI, bool XS>
+template <bool BX4, bool Q4, bool UNI, bool XS, int TT>
 __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
     static_assert(!UNI || BX4, "uniform copies need whole 16-byte stages");
     static_assert(!XS || UNI, "the split layout is copied from uniform bases");
+    using G = GemmTile<TT>;
+    constexpr int T2 = G::T2;
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hi = lane >> 5;
     const int q4_shift = hi ? 0 : 4;
     const int cols = a.cols, nb = a.nb;
-    const int n_tt = (a.n_tok + kGemmToks - 1) / kGemmToks;
+    const int n_tt = (a.n_tok + TT - 1) / TT;
     const int n_rt = (a.rows_total + kGemmRows - 1) / kGemmRows;
     // split ks of ksplit takes the ks-th run of stages; the grid repeats the
     // tile order once per split (a multiple of 8 work-groups each, so the XCD
@@ -514,12 +528,12 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
     const int k = bx >> 3;
     const int rt = (k / n_tt) * 8 + (bx & 7), tt = k % n_tt;
     if (rt >= n_rt) return;   // the padding of the last row of XCD groups
-    const int row0 = rt * kGemmRows, tok0 = tt * kGemmToks;
+    const int row0 = rt * kGemmRows, tok0 = tt * TT;
     const int stages = (nb + kGemmKB - 1) / kGemmKB;
     const int st_begin = ks * stages / a.ksplit, st_end = (ks + 1) * stages / a.ksplit;
-    const int wr = 32 * (wave & 3), wt = 64 * (wave >> 2);
-    // where this wave's 64 token scales of a stage go: block wave / 2, tokens 64 (wave & 1)..
-    const int sdst = 4 * (kGemmScaleRow * (wave >> 1) + 64 * (wave & 1));
+    const int wr = 32 * (wave & 3), wt = 32 * T2 * (wave >> 2);
+    // this wave's token scales of a stage: block, first token
+    const int s_blk = TT == 128 ? wave >> 1 : wave, s_tok = TT == 128 ? 64 * (wave & 1) : 0;
 
     // A: thread tid copies 16 bytes of row tid / 4 (both halves of the block,
     // slot tid % 4); WD: one row's four scales per lane (dwords: scale tid % 4
@@ -550,7 +564,7 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
     const unsigned char *useg = nullptr;   // the rows' segment: codes, then scales at uscale
     const unsigned char *uwd = nullptr;    // the same for this wave's scale rows
     size_t uscale = 0;
-    uint32_t vrow = 0, vdrow = 0, vb[kGemmBRounds];
+    uint32_t vrow = 0, vdrow = 0, vb[XS ? 2 : G::ROUNDS];
     if constexpr (uni) {
         const bool s0 = row0 < a.seg_end[0], s1 = !s0 && row0 < a.seg_end[1];
         useg = uwd = s0 ? a.seg[0].w : (s1 ? a.seg[1].w : a.seg[2].w);
@@ -573,17 +587,17 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         vrow = (uint32_t)r * rowb + 16u * (uint32_t)my_blk;
         vdrow = (uint32_t)rd * (uint32_t)nb * 4u;
         if constexpr (XS) {
-            // every copy of this lane is for token 64 (wave & 1) + lane of the
-            // tile: its 16-byte half-block and its scale in the block-major runs
-            const int tk = 64 * (wave & 1) + lane;
+            // every copy of this lane is for one token of the tile: its
+            // 16-byte half-block and its scale in the block-major runs
+            const int tk = s_tok + lane;
             const int t = tok0 + tk < a.n_tok ? tok0 + tk : a.n_tok - 1;
             vb[0] = 16u * (uint32_t)t;
             vb[1] = 4u * (uint32_t)t;
         } else {
 #pragma unroll
-            for (int j = 0; j < kGemmBRounds; j++) {
+            for (int j = 0; j < G::ROUNDS; j++) {
                 const int c = tid + kGemmThreads * j;
-                const int cc = c < kGemmBChunks ? c : kGemmBChunks - 1;
+                const int cc = c < G::CHUNKS ? c : G::CHUNKS - 1;
                 const int tk = cc / 9, piece = cc - 9 * tk;
                 const int t = tok0 + tk < a.n_tok ? tok0 + tk : a.n_tok - 1;
                 vb[j] = (uint32_t)t * (uint32_t)nb * (uint32_t)kBlockBytes + 16u * (uint32_t)piece;
@@ -593,12 +607,12 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
 
     // The token rows' sources of this thread's B copies, fixed over the stages
     // (a stage only adds 36 bytes per block to each).
-    const unsigned char *bsrc[kGemmBRounds];
+    const unsigned char *bsrc[G::ROUNDS];
     if (BX4) {
 #pragma unroll
-        for (int j = 0; j < kGemmBRounds; j++) {
+        for (int j = 0; j < G::ROUNDS; j++) {
             const int c = tid + kGemmThreads * j;
-            const int cc = c < kGemmBChunks ? c : kGemmBChunks - 1;
+            const int cc = c < G::CHUNKS ? c : G::CHUNKS - 1;
             const int tk = cc / 9, piece = cc - 9 * tk;
             const int t = tok0 + tk < a.n_tok ? tok0 + tk : a.n_tok - 1;
             bsrc[j] = a.xq + (size_t)t * nb * kBlockBytes + 16 * piece;
@@ -630,14 +644,15 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         }
         pd = uwd + uscale + 4 * b0;
         if constexpr (XS) {
-            // codes: chunk c -> (block c / 256, half (c / 128) & 1, token c % 128),
-            // the wave's two: half (wave / 2) & 1 of blocks wave / 4 and 2 + wave / 4;
-            // scales: dword c -> (block c / 128, token c % 128), block wave / 2
+            // codes: 16-byte chunk c -> (block c / 2TT, half (c / TT) & 1,
+            // token c % TT), so the wave's one or two copies are of half
+            // `half` of block blk (and blk + 2); scales: one block's tokens
             const size_t n16 = 16 * (size_t)a.n_tok;
+            const int blk = TT == 128 ? wave >> 2 : wave >> 1, half = TT == 128 ? (wave >> 1) & 1 : wave & 1;
             xstep = 2 * kGemmKB * n16;
-            px[0] = a.xq + (size_t)(2 * (b0 + (wave >> 2)) + ((wave >> 1) & 1)) * n16;
+            px[0] = a.xq + (size_t)(2 * (b0 + blk) + half) * n16;
             px[1] = px[0] + 4 * n16;
-            pxd = a.xq + (size_t)a.n_tok * cols + 4 * (size_t)(b0 + (wave >> 1)) * a.n_tok;
+            pxd = a.xq + (size_t)a.n_tok * cols + 4 * (size_t)(b0 + s_blk) * a.n_tok;
         } else {
             px[0] = a.xq + (size_t)b0 * kBlockBytes;
         }
@@ -649,16 +664,21 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         if (wave < 2) dma16s<kGemmA>(pd, vdrow, at);
         if constexpr (XS) {
             dma16s<kGemmA + kGemmWD>(px[0], vb[0], at);
-            dma16s<kGemmA + kGemmWD + 16 * kGemmThreads>(px[1], vb[0], at);
-            dma4s<kGemmA + kGemmWD + kGemmXsCodes>(pxd, vb[1], buf + sdst);
+            if (TT == 128) dma16s<kGemmA + kGemmWD + 16 * kGemmThreads>(px[1], vb[0], at);
+            if (TT == 128 || wave < kGemmKB)
+                dma4s<kGemmA + kGemmWD + G::CODES>(pxd, vb[1], buf + 4 * (G::SROW * s_blk + s_tok));
             px[0] += xstep;
             px[1] += xstep;
             pxd += xstep / 8;
         } else {
+            // whole rounds, then the waves of the last one
+            constexpr int REST = G::CHUNKS % kGemmThreads / 64;
             dma16s<kGemmA + kGemmWD>(px[0], vb[0], at);
-            dma16s<kGemmA + kGemmWD + 16 * kGemmThreads>(px[0], vb[1], at);
-            static_assert(kGemmBRounds == 3 && kGemmBChunks - 2 * kGemmThreads == 128, "the third round is two waves'");
-            if (wave < 2) dma16s<kGemmA + kGemmWD + 32 * kGemmThreads>(px[0], vb[2], at);
+            if (TT == 128 || wave < REST) dma16s<kGemmA + kGemmWD + 16 * kGemmThreads>(px[0], vb[1], at);
+            if constexpr (TT == 128) {
+                if (wave < REST) dma16s<kGemmA + kGemmWD + 32 * kGemmThreads>(px[0], vb[2], at);
+            }
+            static_assert(G::ROUNDS == (TT == 128 ? 3 : 2), "the rounds above");
             px[0] += kGemmKB * kBlockBytes;
         }
         pd += 4 * kGemmKB;
@@ -693,13 +713,14 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         if (BX4) {
             // the last round's copies past the tile are left out (whole waves)
 #pragma unroll
-            for (int j = 0; j < kGemmBRounds; j++)
-                if (tid + kGemmThreads * j < kGemmBChunks)
+            for (int j = 0; j < G::ROUNDS; j++)
+                if (tid + kGemmThreads * j < G::CHUNKS)
                     dma16(bsrc[j] + b0 * kBlockBytes, buf + kGemmA + kGemmWD + 16 * (tid + kGemmThreads * j - lane));
         } else {
 #pragma unroll
-            for (int j = 0; j < kGemmBWords / kGemmThreads; j++) {
+            for (int j = 0; j < (G::WORDS + kGemmThreads - 1) / kGemmThreads; j++) {
                 const int c = tid + kGemmThreads * j;
+                if (c >= G::WORDS) break;   // whole waves
                 const int tk = c / (kGemmBRow / 4), w = c - tk * (kGemmBRow / 4);
                 const int blk = w / 9;
                 const int t = tok0 + tk < a.n_tok ? tok0 + tk : a.n_tok - 1;
@@ -710,9 +731,9 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         }
     };
 
-    v16f acc[2];
+    v16f acc[T2];
 #pragma unroll
-    for (int t2 = 0; t2 < 2; t2++) acc[t2] = v16f(0.0f);
+    for (int t2 = 0; t2 < T2; t2++) acc[t2] = v16f(0.0f);
 
     // Two buffers (73.7 KB, so two work-groups share a CU): stage st+1 is
     // copied while stage st is multiplied.
@@ -724,14 +745,14 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         issue(st_begin, smem);
     }
     for (int st = st_begin; st < st_end; st++) {
-        unsigned char *buf = smem + ((st - st_begin) & 1) * kGemmStage;
+        unsigned char *buf = smem + ((st - st_begin) & 1) * G::STAGE;
         wait_vm<0>();      // this wave's copies of stage st have landed
         __syncthreads();   // stage st is in LDS everywhere; stage st-1's buffer is free
         if (st + 1 < st_end) {
             if constexpr (uni)
-                issue_uni(lds0 + (((st + 1 - st_begin) & 1) ? kGemmStage : 0));
+                issue_uni(lds0 + (((st + 1 - st_begin) & 1) ? G::STAGE : 0));
             else
-                issue(st + 1, smem + ((st + 1 - st_begin) & 1) * kGemmStage);
+                issue(st + 1, smem + ((st + 1 - st_begin) & 1) * G::STAGE);
         }
         const unsigned char *A = buf, *WD = buf + kGemmA, *B = buf + kGemmA + kGemmWD;
         // the row's four scales (times 1/16 for the Q4 codes, which come as 16 x code)
@@ -741,12 +762,12 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         for (int b2 = 0; b2 < kGemmKB; b2 += 2) {
             // both blocks' scales: lane (l32, hi) holds those of block b2 + hi
             const float wd = b2 == 0 ? (hi ? wd4.y : wd4.x) : (hi ? wd4.w : wd4.z);
-            float xd[2];
+            float xd[T2];
 #pragma unroll
-            for (int t2 = 0; t2 < 2; t2++) {
+            for (int t2 = 0; t2 < T2; t2++) {
                 const int t = wt + 32 * t2 + l32;
                 if constexpr (XS) {
-                    xd[t2] = *reinterpret_cast<const float *>(B + kGemmXsCodes + ((b2 + hi) * kGemmScaleRow + t) * 4);
+                    xd[t2] = *reinterpret_cast<const float *>(B + G::CODES + ((b2 + hi) * G::SROW + t) * 4);
                 } else {
                     // (with 16-byte token rows every stage is whole; past nb the
                     // copies repeat block nb - 1: load and select, no branch)
@@ -754,7 +775,7 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
                     xd[t2] = BX4 || st * kGemmKB + b2 + hi < nb ? xv : 0.0f;
                 }
             }
-            v4i wv[2], xv[2][2];
+            v4i wv[2], xv[2][T2];
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 const int blk = b2 + j;
@@ -767,10 +788,10 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
                         A + ((hi * kGemmRows + wr + l32) * kGemmKB + gemm_slot(blk, wr + l32)) * 16);
                 }
 #pragma unroll
-                for (int t2 = 0; t2 < 2; t2++) {
+                for (int t2 = 0; t2 < T2; t2++) {
                     const int t = wt + 32 * t2 + l32;
                     if constexpr (XS) {
-                        xv[j][t2] = *reinterpret_cast<const v4i *>(B + ((blk * 2 + hi) * kGemmToks + t) * 16);
+                        xv[j][t2] = *reinterpret_cast<const v4i *>(B + ((blk * 2 + hi) * TT + t) * 16);
                     } else {
                         const int *x = reinterpret_cast<const int *>(B + t * kGemmBRow + blk * kBlockBytes + 4 + 16 * hi);
                         xv[j][t2] = v4i{x[0], x[1], x[2], x[3]};
@@ -778,7 +799,7 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
                 }
             }
 #pragma unroll
-            for (int t2 = 0; t2 < 2; t2++) {
+            for (int t2 = 0; t2 < T2; t2++) {
                 const v32f p = __builtin_amdgcn_mfma_f32_32x32x1f32(xd[t2], wd, v32f(0.0f), 0, 0, 0);
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
@@ -802,11 +823,11 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         // written in the split layout (codes of block b, token t at
         // ((2b + half) n + t) 16, scales [b][t] after the n * inter code bytes)
         constexpr int kHs = kGemmRows + 4;
-        static_assert(kGemmToks * kHs * 4 <= kGemmBufs * kGemmStage, "the fp32 tile fits the stage buffers");
+        static_assert(TT * kHs * 4 <= kGemmBufs * G::STAGE, "the fp32 tile fits the stage buffers");
         float *hs = reinterpret_cast<float *>(smem);
         __syncthreads();   // every wave is done with the last stage
 #pragma unroll
-        for (int t2 = 0; t2 < 2; t2++)
+        for (int t2 = 0; t2 < T2; t2++)
 #pragma unroll
             for (int i = 0; i < 16; i++) hs[tok(t2, i) * kHs + wr + l32] = acc[t2][i];
         __syncthreads();
@@ -815,9 +836,9 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         // (block, token) units in block-major order: consecutive units are
         // consecutive tokens, so a wave's code stores are 128 contiguous bytes
 #pragma unroll
-        for (int j = 0; j < 2 * kGemmToks * 8 / kGemmThreads; j++) {
+        for (int j = 0; j < 2 * TT * 8 / kGemmThreads; j++) {
             const int q = tid + kGemmThreads * j;
-            const int e = q & 7, bl = q >> 10, tk = (q >> 3) & (kGemmToks - 1);
+            const int e = q & 7, bl = q / (8 * TT), tk = (q >> 3) & (TT - 1);
             const int t = tok0 + tk;
             if (t >= n) continue;   // whole 8-lane groups share t
             const float4 g4 = *reinterpret_cast<const float4 *>(hs + tk * kHs + 32 * bl + 4 * e);
@@ -842,7 +863,7 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         ldy = s0 ? a.seg[0].rows : (s1 ? a.seg[1].rows : a.seg[2].rows);
     }
 #pragma unroll
-    for (int t2 = 0; t2 < 2; t2++)
+    for (int t2 = 0; t2 < T2; t2++)
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const int t = tok0 + tok(t2, i);
@@ -851,18 +872,77 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
 }
 
 // The split-K sum: y of (token t, row r) is the splits' partials added in
-// split order (the same order on every launch).
+// split order (the same order on every launch).  VEC: four rows per thread
+// (every segment's rows a multiple of 4, 16-byte aligned partials and
+// outputs); the loads of four splits are in flight together.  Bound by those
+// loads' latency: 16 splits of 100 x 4,096 (26 MB) took 7.1 us a row per
+// thread, one split after another.
+template <bool VEC>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemvArgs a) {
+    typedef float vec_t __attribute__((ext_vector_type(VEC ? 4 : 1)));
+    constexpr int W = VEC ? 4 : 1;
     const size_t total = (size_t)a.n_tok * a.rows_total;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
-        float acc = a.part[i];
-        for (int s = 1; s < a.ksplit; s++) acc += a.part[(size_t)s * total + i];
+    for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * W; i < total; i += (size_t)gridDim.x * 256 * W) {
+        const float *p = a.part + i;
+        vec_t acc = *reinterpret_cast<const vec_t *>(p);
+        int s = 1;
+        for (; s + 4 <= a.ksplit; s += 4) {
+            vec_t v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = *reinterpret_cast<const vec_t *>(p + (size_t)(s + k) * total);
+#pragma unroll
+            for (int k = 0; k < 4; k++) acc += v[k];
+        }
+        for (; s < a.ksplit; s++) acc += *reinterpret_cast<const vec_t *>(p + (size_t)s * total);
         const int t = (int)(i / a.rows_total), r = (int)(i - (size_t)t * a.rows_total);
         const bool s0 = r < a.seg_end[0], s1 = !s0 && r < a.seg_end[1];
         float *y = s0 ? a.seg[0].y : (s1 ? a.seg[1].y : a.seg[2].y);
         const int rows = s0 ? a.seg[0].rows : (s1 ? a.seg[1].rows : a.seg[2].rows);
         const int lr = r - (s0 ? 0 : (s1 ? a.seg_end[0] : a.seg_end[1]));
-        y[(size_t)t * rows + lr] = acc;
+        *reinterpret_cast<vec_t *>(y + (size_t)t * rows + lr) = acc;
+    }
+}
+
+// The split-K sum of the MLP's gate and up matmul and silu_quant8_kernel's
+// work in one launch: thread (token, block, lane of 8) adds four gate and four
+// up values' partials in split order, stores them, forms h = silu(g) * u and
+// quantizes the block with its 7 neighbours, into the split layout (a.hq_xs)
+// or block_q8 rows at a.hq.  The same values as the two launches, without the
+// second's launch and read.  seg[0].y and seg[1].y 16-byte aligned.
+__global__ __launch_bounds__(256) void gemm_reduce_silu_kernel(GemvArgs a) {
+    const int inter = a.seg[0].rows, nbi = inter / kQK, n = a.n_tok;
+    const size_t k = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= (size_t)n * nbi * 8) return;   // whole 8-lane groups
+    const int e = (int)(k & 7);
+    const size_t tb = k >> 3;
+    const int t = (int)(tb / nbi), b = (int)(tb - (size_t)t * nbi);
+    const size_t total = (size_t)n * a.rows_total;
+    const float *pg = a.part + (size_t)t * a.rows_total + kQK * b + 4 * e, *pu = pg + inter;
+    v4f g = *reinterpret_cast<const v4f *>(pg), u = *reinterpret_cast<const v4f *>(pu);
+    int s = 1;
+    for (; s + 2 <= a.ksplit; s += 2) {
+        const v4f g0 = *reinterpret_cast<const v4f *>(pg + s * total), u0 = *reinterpret_cast<const v4f *>(pu + s * total);
+        const v4f g1 = *reinterpret_cast<const v4f *>(pg + (s + 1) * total);
+        const v4f u1 = *reinterpret_cast<const v4f *>(pu + (s + 1) * total);
+        g += g0;
+        u += u0;
+        g += g1;
+        u += u1;
+    }
+    if (s < a.ksplit) {
+        g += *reinterpret_cast<const v4f *>(pg + s * total);
+        u += *reinterpret_cast<const v4f *>(pu + s * total);
+    }
+    const size_t at = (size_t)t * inter + kQK * b + 4 * e;
+    *reinterpret_cast<v4f *>(a.seg[0].y + at) = g;
+    *reinterpret_cast<v4f *>(a.seg[1].y + at) = u;
+    const float h[4] = {silu_mul(g.x, u.x), silu_mul(g.y, u.y), silu_mul(g.z, u.z), silu_mul(g.w, u.w)};
+    if (a.hq_xs) {
+        float *scales = reinterpret_cast<float *>(a.hq + (size_t)n * inter);
+        quantize8x4(h, scales + (size_t)b * n + t, a.hq + ((size_t)(2 * b + (e >> 2)) * n + t) * 16 + 4 * (e & 3), e == 0);
+    } else {
+        unsigned char *blk = a.hq + tb * kBlockBytes;
+        quantize8x4(h, reinterpret_cast<float *>(blk), blk + 4 + 4 * e, e == 0);
     }
 }
 
@@ -953,21 +1033,28 @@ hipError_t launch_gemv(const GemvArgs &a, int tcap, bool xf, int rw, int gc, hip
     }
 }
 
-// From how many tokens on (block_q8 input) the MFMA GEMM runs instead of GEMV
-// launches of tmax tokens each (TQ_HIP_GEMM_MIN_TOKENS overrides).  A GEMV
-// launch streams the weights once (about 5 TB/s, plus 2 us of launch), so
-// its cost grows with the token count; the GEMM's first round of 128-row
-// tiles costs its K loop, about 0.0183 us per column on MI355X, whatever the
-// token count.  Measured crossovers: 6144 x 4096 between 64 and 96 tokens
-// (77 against 62 us at 64), 28672 x 4096 between 16 and 32, 4096 x 14336
-// between 64 and 96; the model below puts them at 80, 22 and 70.
+// One GEMV launch of up to tmax tokens streams the weights once, at about
+// 5 TB/s of Q8 bytes (Q4 launches of 8 tokens take as long: their vector work
+// is the same), plus its launch.
+double gemv_us(int rows, int cols) { return (double)rows * cols * (kBlockBytes / (double)kQK) / 5.0e6 + 2.5; }
+
+// From how many tokens on (block_q8 input) the unsplit MFMA GEMM runs instead
+// of GEMV launches of tmax tokens each (TQ_HIP_GEMM_MIN_TOKENS overrides).
+// GEMV's cost grows with the token count; the GEMM's first round of 128-row
+// tiles costs its K loop: measured 0.0072 us per column with 64-token tiles
+// and 0.0133 with 128-token ones.  us, GEMM against GEMV launches:
+//   6144 x 4096    16 tokens 33 / 18    32: 33 / 33    64: 34 / 63    96: 58 / 94
+//   28672 x 4096    8: 48 / 35    12: 48 / 55    32: 48 / 121    96: 68 / 346
+//   4096 x 14336   16: 105 / 58   32: 105 / 116  64: 106 / 231   96: 190 / 345
+// The model puts the crossovers at 33, 16 (the least) and 28.
 int gemm_min_tokens(int rows, int cols, int tmax) {
     const int v = env_int("TQ_HIP_GEMM_MIN_TOKENS", 0);
     if (v > 0) return v;
-    const double chunk_us = (double)rows * cols * (kBlockBytes / (double)kQK) / 5.0e6 + 2.0;
-    const double gemm_us = 0.0183 * cols + 2.0;
-    const int n = (int)(tmax * gemm_us / chunk_us) + 1;
-    return n < 16 ? 16 : (n > 256 ? 256 : n);
+    const double per_token = gemv_us(rows, cols) / tmax;
+    const int n64 = (int)((0.0072 * cols + 3.5) / per_token) + 1;
+    if (n64 <= 64) return n64 < 16 ? 16 : n64;   // up to 15 tokens a row's bits are the GEMV's whatever its batch
+    const int n128 = (int)((0.0133 * cols + 3.5) / per_token) + 1;
+    return n128 < 65 ? 65 : (n128 > 256 ? 256 : n128);
 }
 
 // Every 128-row tile inside one segment (segment ends on tile boundaries) and
@@ -981,79 +1068,105 @@ bool gemm_uniform(const GemvArgs &a) {
     return (size_t)a.n_tok * a.nb * kBlockBytes < ((size_t)1 << 31);
 }
 
+// Tokens per tile of a launch over n_tok: 64 where one such tile holds them.
+int gemm_toks(int n_tok) { return n_tok <= 64 ? 64 : 128; }
+
+template <int TT>
+hipError_t launch_gemm_t(const GemvArgs &u, bool bx4, unsigned grid, hipStream_t s) {
+    const size_t lds = (size_t)kGemmBufs * GemmTile<TT>::STAGE;
+    if (lds > kDefaultLdsLimit) {
+        static bool opted = false;   // once per tile (and process)
+        if (!opted) {
+            for (const void *f : {(const void *)gemm_q8_kernel<true, false, false, false, TT>,
+                                  (const void *)gemm_q8_kernel<false, false, false, false, TT>,
+                                  (const void *)gemm_q8_kernel<true, true, false, false, TT>,
+                                  (const void *)gemm_q8_kernel<false, true, false, false, TT>,
+                                  (const void *)gemm_q8_kernel<true, false, true, false, TT>,
+                                  (const void *)gemm_q8_kernel<true, true, true, false, TT>,
+                                  (const void *)gemm_q8_kernel<true, false, true, true, TT>,
+                                  (const void *)gemm_q8_kernel<true, true, true, true, TT>}) {
+                const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                if (e != hipSuccess) return e;
+            }
+            opted = true;
+        }
+    }
+    const dim3 g(grid), b(kGemmThreads);
+    if (u.q4) {
+        if (u.xs)
+            hipLaunchKernelGGL((gemm_q8_kernel<true, true, true, true, TT>), g, b, lds, s, u);
+        else if (bx4 && u.uni_tiles)
+            hipLaunchKernelGGL((gemm_q8_kernel<true, true, true, false, TT>), g, b, lds, s, u);
+        else if (bx4)
+            hipLaunchKernelGGL((gemm_q8_kernel<true, true, false, false, TT>), g, b, lds, s, u);
+        else
+            hipLaunchKernelGGL((gemm_q8_kernel<false, true, false, false, TT>), g, b, lds, s, u);
+    } else {
+        if (u.xs)
+            hipLaunchKernelGGL((gemm_q8_kernel<true, false, true, true, TT>), g, b, lds, s, u);
+        else if (bx4 && u.uni_tiles)
+            hipLaunchKernelGGL((gemm_q8_kernel<true, false, true, false, TT>), g, b, lds, s, u);
+        else if (bx4)
+            hipLaunchKernelGGL((gemm_q8_kernel<true, false, false, false, TT>), g, b, lds, s, u);
+        else
+            hipLaunchKernelGGL((gemm_q8_kernel<false, false, false, false, TT>), g, b, lds, s, u);
+    }
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm(const GemvArgs &a, int ksplit, hipStream_t s) {
+    const int toks = gemm_toks(a.n_tok);
     const int n_rt = (a.rows_total + kGemmRows - 1) / kGemmRows;
-    const int n_tt = (a.n_tok + kGemmToks - 1) / kGemmToks;
+    const int n_tt = (a.n_tok + toks - 1) / toks;
     const long groups = ((long)n_rt + 7) / 8;   // row tiles per XCD, rounded up
     const long grid = groups * 8 * n_tt * ksplit;
     if (grid > INT32_MAX) return hipErrorInvalidValue;
-    const size_t lds = (size_t)kGemmBufs * kGemmStage;
-    static bool opted = false;
-    if (!opted) {
-        for (const void *f : {(const void *)gemm_q8_kernel<true, false, false, false>,
-                              (const void *)gemm_q8_kernel<false, false, false, false>,
-                              (const void *)gemm_q8_kernel<true, true, false, false>,
-                              (const void *)gemm_q8_kernel<false, true, false, false>,
-                              (const void *)gemm_q8_kernel<true, false, true, false>,
-                              (const void *)gemm_q8_kernel<true, true, true, false>,
-                              (const void *)gemm_q8_kernel<true, false, true, true>,
-                              (const void *)gemm_q8_kernel<true, true, true, true>}) {
-            const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-        }
-        opted = true;
-    }
     const bool bx4 = (((uintptr_t)a.xq & 15) == 0) && a.nb % kGemmKB == 0;
     GemvArgs u = a;
     u.ksplit = ksplit;
     u.uni_tiles = gemm_uniform(a);
     if (a.xs && !(bx4 && u.uni_tiles)) return hipErrorInvalidValue;   // the caller's plan and this disagree
-    // paired gate/up tiles: one unsplit split-layout GEMM over two segments
-    // of equal rows, a multiple of 64
-    if (a.hq && (ksplit != 1 || !a.xs || a.seg[0].rows != a.seg[1].rows || a.seg[0].rows % 64 != 0 ||
-                 a.rows_total != 2 * a.seg[0].rows))
+    // the hidden rows instead of gate and up: two segments of equal rows; in
+    // paired tiles (unsplit) a split-layout GEMM and rows a multiple of 64
+    if (a.hq && (a.seg[0].rows != a.seg[1].rows || a.rows_total != 2 * a.seg[0].rows ||
+                 (ksplit == 1 ? !a.xs || !a.hq_xs || a.seg[0].rows % 64 != 0 : a.seg[0].rows % kQK != 0)))
         return hipErrorInvalidValue;
-    const dim3 g((unsigned)grid), b(kGemmThreads);
-    if (a.q4) {
-        if (a.xs)
-            hipLaunchKernelGGL((gemm_q8_kernel<true, true, true, true>), g, b, lds, s, u);
-        else if (bx4 && u.uni_tiles)
-            hipLaunchKernelGGL((gemm_q8_kernel<true, true, true, false>), g, b, lds, s, u);
-        else if (bx4)
-            hipLaunchKernelGGL((gemm_q8_kernel<true, true, false, false>), g, b, lds, s, u);
-        else
-            hipLaunchKernelGGL((gemm_q8_kernel<false, true, false, false>), g, b, lds, s, u);
-    } else {
-        if (a.xs)
-            hipLaunchKernelGGL((gemm_q8_kernel<true, false, true, true>), g, b, lds, s, u);
-        else if (bx4 && u.uni_tiles)
-            hipLaunchKernelGGL((gemm_q8_kernel<true, false, true, false>), g, b, lds, s, u);
-        else if (bx4)
-            hipLaunchKernelGGL((gemm_q8_kernel<true, false, false, false>), g, b, lds, s, u);
-        else
-            hipLaunchKernelGGL((gemm_q8_kernel<false, false, false, false>), g, b, lds, s, u);
+    if (ksplit > 1) u.hq = nullptr;   // the reduce launch's
+    const hipError_t e = toks == 64 ? launch_gemm_t<64>(u, bx4, (unsigned)grid, s)
+                                    : launch_gemm_t<128>(u, bx4, (unsigned)grid, s);
+    if (e != hipSuccess || ksplit == 1) return e;
+    u.hq = a.hq;
+    const size_t total = (size_t)a.n_tok * a.rows_total;
+    if (u.hq) {
+        const size_t threads = (size_t)a.n_tok * (a.seg[0].rows / kQK) * 8;
+        hipLaunchKernelGGL(gemm_reduce_silu_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, u);
+        return hipGetLastError();
     }
-    if (ksplit > 1) {
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        const size_t total = (size_t)a.n_tok * a.rows_total;
-        const size_t blocks = (total + 255) / 256 < 2048 ? (total + 255) / 256 : 2048;
-        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, u);
-    }
+    bool vec = ((uintptr_t)a.part & 15) == 0;
+    for (int i = 0; i < kMaxSegs; i++)
+        vec = vec && (((uintptr_t)a.seg[i].y & 15) == 0) && a.seg[i].rows % 4 == 0 && a.seg_end[i] % 4 == 0;
+    const size_t per = vec ? 4 : 1;
+    const size_t blocks = std::min<size_t>((total / per + 255) / 256, 2048);
+    if (vec)
+        hipLaunchKernelGGL(gemm_reduce_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, s, u);
+    else
+        hipLaunchKernelGGL(gemm_reduce_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, s, u);
     return hipGetLastError();
 }
 
 // Split-K GEMM while the tiles alone leave CUs of the 256 idle (each tile
 // then runs the whole K loop): K is cut into S runs of stages, as many as
 // keep the grid within one round of 512 work-groups (two per CU), each split
-// writing a partial tile that one more launch sums in split order.  The 8B
-// MLP over 16 / 64 / 256 / 512 rows: 130 / 141 / 272 / 481 us against
-// 134 / 325 / 427 / 570 without.
+// writing a partial tile that one more launch sums in split order.  MLP at
+// the 8B shape, us with Q8 / Q4 weights over 9, 16, 64, 100, 256 rows:
+// 72 / 59, 74 / 58, 84 / 70, 106 / 98, 158 / 154; before 64-token tiles and
+// with 16 tokens as the least, 100 / 76, 96 / 88, 105 / 97, 114 / 105, 164 / 157.
 constexpr int kSplitWgs = 512;
+constexpr int kSplitMinTokens = 9;
 
 int gemm_ksplit(int rows, int cols, int n_tok) {
-    if (n_tok < 16) return 1;
-    const long wgs = ((long)(rows + kGemmRows - 1) / kGemmRows + 7) / 8 * 8 * ((n_tok + kGemmToks - 1) / kGemmToks);
+    if (n_tok < kSplitMinTokens) return 1;
+    const long wgs = ((long)(rows + kGemmRows - 1) / kGemmRows + 7) / 8 * 8 * ((n_tok + gemm_toks(n_tok) - 1) / gemm_toks(n_tok));
     // once every CU holds a tile, splitting adds occupancy but not CUs, and
     // the partials' traffic outweighs it (4,096 x 14,336 at 1,024 tokens)
     if (wgs >= kSplitWgs / 2) return 1;
@@ -1069,10 +1182,19 @@ int gemm_ksplit(int rows, int cols, int n_tok) {
 int gemm_plan(const GemvArgs &a, int n_tok) {
     if (a.x != nullptr) return 0;
     const int ksplit = a.part ? gemm_ksplit(a.rows_total, a.cols, n_tok) : 1;
-    const bool split = ksplit > 1 && (size_t)ksplit * n_tok * a.rows_total <= a.part_floats &&
-                       env_int("TQ_HIP_GEMM_SPLIT", 1) != 0;
+    const int tmax = pick_tokens(a.nb, false);
+    bool split = ksplit > 1 && (size_t)ksplit * n_tok * a.rows_total <= a.part_floats &&
+                 env_int("TQ_HIP_GEMM_SPLIT", 1) != 0;
+    // 9-15 tokens: the split GEMM and its reduce (about 3.6 TB/s of the
+    // weights and 8 us) where the two or more GEMV launches take longer (8B:
+    // gate/up 42 against 55 us at 12 tokens, down 24 against 44; q/k/v and
+    // output stay with GEMV, 15 and 13)
+    if (split && n_tok < 16 && tmax > 0) {
+        const double bytes = (double)a.rows_total * a.nb * (a.q4 ? kBlockBytes4 : kBlockBytes);
+        split = bytes / 3.6e6 + 8.0 < (n_tok + tmax - 1) / tmax * gemv_us(a.rows_total, a.cols);
+    }
     if (split) return ksplit;
-    return n_tok >= gemm_min_tokens(a.rows_total, a.cols, pick_tokens(a.nb, false)) ? 1 : 0;
+    return n_tok >= gemm_min_tokens(a.rows_total, a.cols, tmax) ? 1 : 0;
 }
 
 // Whether the matmul's input should be quantized into the split layout:
@@ -1340,10 +1462,10 @@ int tq_project_output_xs(bool q4, const void *wo, int rows, int cols, const void
 // Partial floats a split-K GEMM of rows x cols needs for any token count up
 // to n_cap: the largest S * n over the token-tile counts that still split.
 size_t tq_gemm_partial_floats(int rows, int cols, int n_cap) {
-    if (rows <= 0 || cols <= 0 || n_cap < 16) return 0;
+    if (rows <= 0 || cols <= 0 || n_cap < kSplitMinTokens) return 0;
     size_t most = 0;
-    for (int tiles = 1; (long)(tiles - 1) * kGemmToks < n_cap; tiles++) {
-        const int n = n_cap < tiles * kGemmToks ? n_cap : tiles * kGemmToks;
+    for (int tiles = 1; (long)(tiles - 1) * 128 < n_cap; tiles++) {
+        const int n = n_cap < tiles * 128 ? n_cap : tiles * 128;
         const int sp = gemm_ksplit(rows, cols, n);
         if (sp < 2) break;
         const size_t need = (size_t)sp * n * rows;
@@ -1390,7 +1512,9 @@ int tq_hip_mlp_layer_async(const tq_hip_mlp_weights *w, int n, const float *d_xn
         !aligned(d_out, 4))
         return TQ_HIP_EINVAL;
     size_t og, ou, ox, op, pf;
-    if (ws_bytes < mlp_ws(w->hidden, w->inter, n, &og, &ou, &ox, &op, &pf)) return TQ_HIP_EINVAL;
+    const size_t full = mlp_ws(w->hidden, w->inter, n, &og, &ou, &ox, &op, &pf);
+    if (ws_bytes < (n < 16 ? op : full)) return TQ_HIP_EINVAL;
+    if (ws_bytes < full) pf = 0;   // 9-15 rows without room for partials: no K splits
     unsigned char *ws = (unsigned char *)d_ws;
     float *gate = (float *)(ws + og), *up = (float *)(ws + ou);
     float *part = (float *)(ws + op);
@@ -1419,24 +1543,28 @@ int tq_hip_mlp_layer_async(const tq_hip_mlp_weights *w, int n, const float *d_xn
     d.rows_total = w->hidden;
     d.part = part;
     d.part_floats = pf;
-    // When the gate/up matmul is one unsplit GEMM over the split layout and
-    // the down matmul reads the split layout too, the gate/up tiles pair 64
-    // rows of both matrices and their epilogue writes the quantized hidden
-    // rows (into the gate rows' space, which they then no longer need);
-    // otherwise gate and up rows go to the workspace and one more launch
-    // forms them (block_q8 rows, or the split layout).  TQ_HIP_MLP_FUSED=0
-    // keeps the separate launch.
-    const bool fused = a.xs && gemm_plan(a, n) == 1 && xs_layout(d, n, gate) &&
-                       env_int("TQ_HIP_MLP_FUSED", 1) != 0;
-    if (fused) a.hq = (unsigned char *)gate;
+    // Where the gate/up matmul is a GEMM it leaves the quantized hidden rows
+    // itself.  Unsplit over the split layout, when the down matmul reads the
+    // split layout too: its tiles pair 64 rows of both matrices and their
+    // epilogue writes them (into the gate rows' space; no gate and up rows).
+    // Split: its reduce launch writes them beside gate and up, in the layout
+    // the down matmul reads, over the quantized input.  Otherwise one more
+    // launch forms them.  TQ_HIP_MLP_FUSED=0 keeps that launch.
+    const bool fuse = env_int("TQ_HIP_MLP_FUSED", 1) != 0;
+    const int plan = gemm_plan(a, n);
+    const bool fused = fuse && a.xs && plan == 1 && w->inter % 64 == 0 && xs_layout(d, n, gate);
+    const bool fused_split = fuse && plan > 1;
+    d.xs = fused || xs_layout(d, n, xq);
+    if (fused || fused_split) {
+        a.hq = fused ? (unsigned char *)gate : (unsigned char *)xq;
+        a.hq_xs = d.xs;
+    }
     rc = run_gemv(a, n, s);
     if (rc != TQ_HIP_OK) return rc;
-    if (fused) {
-        d.xs = true;
-        d.xq = (const unsigned char *)gate;
+    if (fused || fused_split) {
+        d.xq = a.hq;
         return run_gemv(d, n, s);
     }
-    d.xs = xs_layout(d, n, xq);
     const hipError_t e = d.xs ? tq_launch_silu_quant_split(gate, up, (unsigned char *)xq, n, w->inter, s)
                               : tq_launch_silu_quant(gate, up, xq, (long)n * w->inter, s);
     if (e != hipSuccess) return herr(e);
