@@ -1379,7 +1379,7 @@ int quantize_input(GemvArgs &a, const float *x, int n_tok, int cols, void *xq_ws
         a.xq_out = (unsigned char *)xq_ws;
         return TQ_HIP_OK;
     }
-    a.xs = xs_layout(a, n_tok, xq_ws);
+    a.xs = aligned(x, 16) && xs_layout(a, n_tok, xq_ws);   // its quantizer loads 16 bytes
     const hipError_t e = a.xs ? tq_launch_quantize_split(x, (unsigned char *)xq_ws, n_tok, cols, s)
                               : tq_launch_quantize(x, (block_q8 *)xq_ws, n_tok * cols, s);
     if (e != hipSuccess) return herr(e);

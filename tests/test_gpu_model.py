@@ -252,6 +252,29 @@ def test_mlp_layer_split_fused(nat, oracle, fmt, hidden, inter, n, monkeypatch):
         assert rel_l2(out1, np.frombuffer(seen[0][0], np.float32)) <= 1e-3
 
 
+@pytest.mark.parametrize("hidden,inter,n", [(4096, 4096, 12), (512, 1024, 20), (512, 1024, 130), (512, 1024, 300)])
+def test_mlp_layer_unaligned_rows(nat, oracle, hidden, inter, n):
+    """xn 4 bytes past a 16-byte boundary where the GEMM would take the split
+    layout (quantized in 16-byte loads): block_q8 rows instead, the same bits.
+    The row counts cover a part of, one and several of the split quantizer's
+    128-row runs."""
+    lib = nat.load()
+    rng = np.random.default_rng(hidden + n)
+    mats = [tiled(nat, oracle.pack_matrix_q8(rng.standard_normal((r, c)).astype(np.float32) * 0.1), r, c)
+            for r, c in ((inter, hidden), (inter, hidden), (hidden, inter))]
+    w = nat.MlpWeights(*(m.ptr for m in mats), hidden, inter)
+    wsb = lib.tq_hip_mlp_ws_bytes(C.byref(w), n)
+    ws, dout = nat.DeviceBuffer(wsb), nat.DeviceBuffer(n * hidden * 4)
+    xn = normal(n * hidden, 11) * 2
+    outs = []
+    for skew in (0, 4):
+        dx = dev(nat, np.concatenate([np.zeros(skew // 4, np.float32), xn]))
+        nat.check(lib.tq_hip_mlp_layer_async(C.byref(w), n, dx.ptr + skew, dout.ptr, ws.ptr, wsb, None), "mlp")
+        sync(nat)
+        outs.append(dout.download((n, hidden), np.float32))
+    assert outs[0].tobytes() == outs[1].tobytes()
+
+
 def test_add_rmsnorm(nat, oracle):
     lib = nat.load()
     # 1024-thread kernel holding 1, 2, 4 and 8 float4 per thread, and the
