@@ -1183,16 +1183,16 @@ int gemm_plan(const GemvArgs &a, int n_tok) {
     if (a.x != nullptr) return 0;
     const int ksplit = a.part ? gemm_ksplit(a.rows_total, a.cols, n_tok) : 1;
     const int tmax = pick_tokens(a.nb, false);
-    bool split = ksplit > 1 && (size_t)ksplit * n_tok * a.rows_total <= a.part_floats &&
-                 env_int("TQ_HIP_GEMM_SPLIT", 1) != 0;
-    // 9-15 tokens: the split GEMM and its reduce (about 3.6 TB/s of the
-    // weights and 8 us) where the two or more GEMV launches take longer (8B:
+    bool split = ksplit > 1 && (size_t)ksplit * n_tok * a.rows_total <= a.part_floats;
+    // 9-15 tokens: the split GEMM and its reduce (about 3.6 TB/s of Q8 bytes,
+    // Q4 matrices 0.8 of that time, and 11 us) where the two or more GEMV launches take longer (8B:
     // gate/up 42 against 55 us at 12 tokens, down 24 against 44; q/k/v and
-    // output stay with GEMV, 15 and 13)
+    // output stay with GEMV: the whole layer 41 us against 44 with the GEMM)
     if (split && n_tok < 16 && tmax > 0) {
-        const double bytes = (double)a.rows_total * a.nb * (a.q4 ? kBlockBytes4 : kBlockBytes);
-        split = bytes / 3.6e6 + 8.0 < (n_tok + tmax - 1) / tmax * gemv_us(a.rows_total, a.cols);
+        const double bytes = (double)a.rows_total * a.nb * kBlockBytes;
+        split = (a.q4 ? 0.8 : 1.0) * bytes / 3.6e6 + 11.0 < (n_tok + tmax - 1) / tmax * gemv_us(a.rows_total, a.cols);
     }
+    split = split && env_int("TQ_HIP_GEMM_SPLIT", 1) != 0;
     if (split) return ksplit;
     return n_tok >= gemm_min_tokens(a.rows_total, a.cols, tmax) ? 1 : 0;
 }
@@ -1550,8 +1550,8 @@ int tq_hip_mlp_layer_async(const tq_hip_mlp_weights *w, int n, const float *d_xn
     // Split: its reduce launch writes them beside gate and up, in the layout
     // the down matmul reads, over the quantized input.  Otherwise one more
     // launch forms them.  TQ_HIP_MLP_FUSED=0 keeps that launch.
-    const bool fuse = env_int("TQ_HIP_MLP_FUSED", 1) != 0;
-    const int plan = gemm_plan(a, n);
+    const int plan = n < kSplitMinTokens ? 0 : gemm_plan(a, n);
+    const bool fuse = plan > 0 && env_int("TQ_HIP_MLP_FUSED", 1) != 0;
     const bool fused = fuse && a.xs && plan == 1 && w->inter % 64 == 0 && xs_layout(d, n, gate);
     const bool fused_split = fuse && plan > 1;
     d.xs = fused || xs_layout(d, n, xq);
