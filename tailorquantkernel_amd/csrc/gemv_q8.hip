@@ -448,9 +448,9 @@ size_t lds_bytes(int t, int nb, bool xf) {
 // shape matters: a wave's weight copy reads 64 contiguous bytes per row (four
 // lanes a row; one lane a row, 16 bytes every row pitch, cost 20 % more).
 // Against 16 x 16 products, vector scale multiplies and 16-byte row pieces
-// (8B shapes): MLP over 2,048 rows 1,267 -> 977 us, its Q4 form over 100 rows
-// 145 -> 104 us, the attention layer over 2,048 rows 452 -> 354 us, results
-// unchanged bit for bit.
+// and per-stage copy addresses (8B shapes): MLP over 2,048 rows 1,277 -> 964
+// us, the attention layer over 2,048 rows 451 -> 352 us, results unchanged bit
+// for bit.
 //
 // Tile order: work-groups are dealt to the 8 XCDs round-robin, so the grid is
 // laid out so that every token tile of one row tile runs on the same XCD
@@ -1185,8 +1185,8 @@ int gemm_plan(const GemvArgs &a, int n_tok) {
     const int tmax = pick_tokens(a.nb, false);
     bool split = ksplit > 1 && (size_t)ksplit * n_tok * a.rows_total <= a.part_floats;
     // 9-15 tokens: the split GEMM and its reduce (about 3.6 TB/s of Q8 bytes,
-    // Q4 matrices 0.8 of that time, and 11 us) where the two or more GEMV launches take longer (8B:
-    // gate/up 42 against 55 us at 12 tokens, down 24 against 44; q/k/v and
+    // Q4 matrices 0.8 of that time, and 11 us) where the two or more GEMV
+    // launches take longer (8B: gate/up 42 against 55 us at 12 tokens, down 24 against 44; q/k/v and
     // output stay with GEMV: the whole layer 41 us against 44 with the GEMM)
     if (split && n_tok < 16 && tmax > 0) {
         const double bytes = (double)a.rows_total * a.nb * kBlockBytes;
