@@ -422,7 +422,7 @@ size_t lds_bytes(int t, int nb, bool xf) {
 
 // ---------------------------------------------------------------------------
 // Many tokens: int8 MFMA GEMM.  A work-group of 8 waves computes a 128-row x
-// 128-token tile (TT = 128), or 64 tokens where a launch has no more; wave w
+// 128-token tile (TT = 128), or 64 where that pads less (gemm_toks); wave w
 // owns rows 32(w%4)..+31 of tokens 64(w/4)..+63 (32(w/4)..+31), two 32 x 32
 // tiles (one).  The smaller tile halves the products and the token copies
 // per weight byte: 28,672 x 4,096 over 64 tokens 49 us against 67 with 128
@@ -1068,8 +1068,17 @@ bool gemm_uniform(const GemvArgs &a) {
     return (size_t)a.n_tok * a.nb * kBlockBytes < ((size_t)1 << 31);
 }
 
-// Tokens per tile of a launch over n_tok: 64 where one such tile holds them.
-int gemm_toks(int n_tok) { return n_tok <= 64 ? 64 : 128; }
+// Tokens per tile of a launch over n_tok: 64 where one such tile holds them,
+// and up to 320 tokens where 128-token tiles would be half padding at the end
+// (an odd count of 64s; a 64-token tile takes 0.54 of a 128-token one).  8B
+// MLP, us with 64 / 128, Q8 then Q4: 130 tokens 140 / 155, 131 / 150; 190: 142
+// / 155, 135 / 154; 300: 206 / 225, 206 / 224.  At 420 the gain is gone (277 /
+// 282, 283 / 277) and at 550 it is a loss (371 / 345).  Attention layers: 8B,
+// 129 tokens 98 / 107, 320: 183 / 193; 70B, 320: 308 / 313, Q4 317 / 305 (its
+// 240 tiles of 128 split K in two, 400 of 64 do not: the one shape that lost).
+constexpr int kGemmSmallToks = 320;
+
+int gemm_toks(int n_tok) { return n_tok <= 64 || (n_tok <= kGemmSmallToks && (n_tok + 63) / 64 % 2) ? 64 : 128; }
 
 template <int TT>
 hipError_t launch_gemm_t(const GemvArgs &u, bool bx4, unsigned grid, hipStream_t s) {

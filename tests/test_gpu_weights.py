@@ -211,7 +211,7 @@ def test_gemm_vs_oracle(nat, oracle, rows, cols, n_tok, monkeypatch):
     check_matmul(gpu_matmul(nat, M, xq, n_tok), ref, Wq, xq, rows, cols, n_tok, f"default {rows}x{cols} n_tok={n_tok}")
 
 
-@pytest.mark.parametrize("rows,n_tok", [(1, 1), (31, 33), (32, 32), (33, 31), (97, 65), (129, 127), (160, 129)])
+@pytest.mark.parametrize("rows,n_tok", [(1, 1), (31, 33), (32, 32), (33, 31), (97, 65), (129, 127), (160, 129), (130, 193), (128, 320), (96, 321)])
 @pytest.mark.parametrize("cols", [32, 128, 160, 2176])
 def test_gemm_tile_edges(nat, oracle, rows, n_tok, cols, monkeypatch):
     """The GEMM at the edges of its 32 x 32 tiles and 4-block stages (2176: a
