@@ -168,7 +168,8 @@ __device__ __forceinline__ void split_bf16(const float (&x)[8], v8bf &hi, v8bf &
 typedef __attribute__((address_space(3))) unsigned char lds_u8;
 
 // 16 bytes from each lane's global address into LDS at dst + 16*lane
-// (global_load_lds_dwordx4; M0 holds the LDS byte address and is restored).
+// (global_load_lds_dwordx4; M0 holds the LDS byte address and is restored; a
+// scalar write of M0 needs one wait state before the copy, the s_nop).
 // Issued as inline assembly so that the compiler does not follow every such
 // copy with a full vmcnt(0) wait before LDS accesses: the kernel waits for
 // exactly the copies it needs (wait_copies), counting them in issue order.
@@ -180,7 +181,7 @@ __device__ __forceinline__ void dma16(const void *src, unsigned char *dst) {
     const uint32_t lds = (uint32_t)(uintptr_t)(lds_u8 *)dst;
     uint32_t saved;
     asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\t"
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
         "global_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
         : "=&s"(saved)
         : "v"(src), "s"(lds));
@@ -191,7 +192,7 @@ __device__ __forceinline__ void dma16s(const unsigned char *base, uint32_t off, 
     const uint32_t lds = (uint32_t)(uintptr_t)(lds_u8 *)dst;
     uint32_t saved;
     asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\t"
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
         "global_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
         : "=&s"(saved)
         : "v"(off), "s"(base), "s"(lds));
@@ -201,7 +202,7 @@ __device__ __forceinline__ void dma4s(const unsigned char *base, uint32_t off, u
     const uint32_t lds = (uint32_t)(uintptr_t)(lds_u8 *)dst;
     uint32_t saved;
     asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\t"
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
         "global_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
         : "=&s"(saved)
         : "v"(off), "s"(base), "s"(lds));

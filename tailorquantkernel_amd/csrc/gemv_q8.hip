@@ -184,14 +184,16 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 // 16 bytes from each active lane's global address into LDS at dst + 16*lane
 // (global_load_lds_dwordx4; M0 holds the LDS byte address and is restored;
-// dst must be the same for the whole wave).
+// dst must be the same for the whole wave).  A scalar write of M0 needs one
+// wait state before the copy that reads it, which the compiler does not add
+// inside an asm block: the s_nop here and in the copies below.
 // The memory clobber keeps every later load after it in program order, which
 // the vmcnt arithmetic below relies on.
 __device__ __forceinline__ void dma16(const void *src, unsigned char *dst) {
     const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_u8 *)dst);
     uint32_t saved;
     asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\t"
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
         "global_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
         : "=&s"(saved)
         : "v"(src), "s"(lds)
@@ -211,7 +213,7 @@ __device__ __forceinline__ void dma4(const void *src, unsigned char *dst) {
     const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_u8 *)dst);
     uint32_t saved;
     asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\t"
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
         "global_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
         : "=&s"(saved)
         : "v"(src), "s"(lds)
@@ -224,14 +226,14 @@ __device__ __forceinline__ void dma4(const void *src, unsigned char *dst) {
 // in these kernels uses it).  base and lds are uniform.
 template <int IMM>
 __device__ __forceinline__ void dma16s(const unsigned char *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1"
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
                  : "v"(off), "s"(base), "s"(lds), "n"(IMM)
                  : "m0", "scc", "memory");
 }
 template <int IMM>
 __device__ __forceinline__ void dma4s(const unsigned char *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dword %0, %1"
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                  :
                  : "v"(off), "s"(base), "s"(lds), "n"(IMM)
                  : "m0", "scc", "memory");

@@ -147,14 +147,15 @@ __device__ __forceinline__ float xrow_sum(float x) {
 typedef __attribute__((address_space(3))) unsigned char lds_u8;
 
 // 16 bytes from each lane's global address into LDS at dst + 16*lane
-// (global_load_lds_dwordx4, M0 = LDS byte address, restored after).  Inline
+// (global_load_lds_dwordx4, M0 = LDS byte address, restored after; a scalar
+// write of M0 needs one wait state before the copy, the s_nop).  Inline
 // assembly keeps the compiler from following the copy with a full vmcnt(0)
 // wait before every LDS access; the kernel waits for its copies itself.
 __device__ __forceinline__ void dma16(const void *src, unsigned char *dst) {
     const uint32_t lds = (uint32_t)(uintptr_t)(lds_u8 *)dst;
     uint32_t saved;
     asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\t"
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
         "global_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
         : "=&s"(saved)
         : "v"(src), "s"(lds));
