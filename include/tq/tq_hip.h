@@ -404,8 +404,7 @@ int tq_hip_attention_layer_async(tq_hip_kv *kv, const tq_hip_attn_weights *w, in
 
 /* attention_layer_batch (model/attention_layer.c:200-243) for tokens
  * pos0..pos0+n-1 of sequence `seq`, all on the device: project_qkv over the n
- * rows of d_xn [n][hidden] (the MFMA GEMM from 16 rows on, or from 9 where
- * its model is the faster), the per-head
+ * rows of d_xn [n][hidden] (the MFMA GEMM from 16 rows on), the per-head
  * RMSNorm of q and k (tq_hip_rmsnorm_rows), RoPE + KV append + causal
  * attention (tq_hip_prefill_async; d_cos/d_sin [n][head_dim/2] or NULL),
  * project_output into d_out [n][hidden].  Where the prefill runs its dense

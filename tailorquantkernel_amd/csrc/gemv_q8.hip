@@ -1169,11 +1169,13 @@ hipError_t launch_gemm(const GemvArgs &a, int ksplit, hipStream_t s) {
 // then runs the whole K loop): K is cut into S runs of stages, as many as
 // keep the grid within one round of 512 work-groups (two per CU), each split
 // writing a partial tile that one more launch sums in split order.  MLP at
-// the 8B shape, us with Q8 / Q4 weights over 9, 16, 64, 100, 256 rows:
-// 72 / 59, 74 / 58, 84 / 70, 106 / 98, 158 / 154; before 64-token tiles and
-// with 16 tokens as the least, 100 / 76, 96 / 88, 105 / 97, 114 / 105, 164 / 157.
+// the 8B shape, us with Q8 / Q4 weights over 16, 64, 100, 256 rows: 74 / 58,
+// 84 / 70, 106 / 98, 158 / 154; before 64-token tiles 96 / 88, 105 / 97,
+// 114 / 105, 164 / 157.  The least is 16 tokens, as without a workspace: up to
+// 15 a row's bits are the GEMV's whatever its batch.  (Splits from 9 tokens
+// took 72 / 59 for 100 / 76 us of GEMV launches there, with other bits.)
 constexpr int kSplitWgs = 512;
-constexpr int kSplitMinTokens = 9;
+constexpr int kSplitMinTokens = 16;
 
 int gemm_ksplit(int rows, int cols, int n_tok) {
     if (n_tok < kSplitMinTokens) return 1;
@@ -1193,19 +1195,9 @@ int gemm_ksplit(int rows, int cols, int n_tok) {
 int gemm_plan(const GemvArgs &a, int n_tok) {
     if (a.x != nullptr) return 0;
     const int ksplit = a.part ? gemm_ksplit(a.rows_total, a.cols, n_tok) : 1;
-    const int tmax = pick_tokens(a.nb, false);
-    bool split = ksplit > 1 && (size_t)ksplit * n_tok * a.rows_total <= a.part_floats;
-    // 9-15 tokens: the split GEMM and its reduce (about 3.6 TB/s of Q8 bytes,
-    // Q4 matrices 0.8 of that time, and 11 us) where the two or more GEMV
-    // launches take longer (8B: gate/up 42 against 55 us at 12 tokens, down 24 against 44; q/k/v and
-    // output stay with GEMV: the whole layer 41 us against 44 with the GEMM)
-    if (split && n_tok < 16 && tmax > 0) {
-        const double bytes = (double)a.rows_total * a.nb * kBlockBytes;
-        split = (a.q4 ? 0.8 : 1.0) * bytes / 3.6e6 + 11.0 < (n_tok + tmax - 1) / tmax * gemv_us(a.rows_total, a.cols);
-    }
-    split = split && env_int("TQ_HIP_GEMM_SPLIT", 1) != 0;
-    if (split) return ksplit;
-    return n_tok >= gemm_min_tokens(a.rows_total, a.cols, tmax) ? 1 : 0;
+    if (ksplit > 1 && (size_t)ksplit * n_tok * a.rows_total <= a.part_floats && env_int("TQ_HIP_GEMM_SPLIT", 1) != 0)
+        return ksplit;
+    return n_tok >= gemm_min_tokens(a.rows_total, a.cols, pick_tokens(a.nb, false)) ? 1 : 0;
 }
 
 // Whether the matmul's input should be quantized into the split layout:
@@ -1523,9 +1515,7 @@ int tq_hip_mlp_layer_async(const tq_hip_mlp_weights *w, int n, const float *d_xn
         !aligned(d_out, 4))
         return TQ_HIP_EINVAL;
     size_t og, ou, ox, op, pf;
-    const size_t full = mlp_ws(w->hidden, w->inter, n, &og, &ou, &ox, &op, &pf);
-    if (ws_bytes < (n < 16 ? op : full)) return TQ_HIP_EINVAL;
-    if (ws_bytes < full) pf = 0;   // 9-15 rows without room for partials: no K splits
+    if (ws_bytes < mlp_ws(w->hidden, w->inter, n, &og, &ou, &ox, &op, &pf)) return TQ_HIP_EINVAL;
     unsigned char *ws = (unsigned char *)d_ws;
     float *gate = (float *)(ws + og), *up = (float *)(ws + ou);
     float *part = (float *)(ws + op);

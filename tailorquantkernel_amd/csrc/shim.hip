@@ -1181,9 +1181,7 @@ int tq_hip_attention_layer_async(tq_hip_kv *kv, const tq_hip_attn_weights *w, in
         return TQ_HIP_EINVAL;
     const tq_hip_kv_desc &D = kv->desc;
     size_t oq, ok, ov, oa, ox, op, pf;
-    const size_t full = layer_ws(D, w->hidden, n_q, &oq, &ok, &ov, &oa, &ox, &op, &pf);
-    if (ws_bytes < (n_q < 16 ? op : full)) return TQ_HIP_EINVAL;
-    if (ws_bytes < full) pf = 0;   // 9-15 rows without room for partials: no K splits
+    if (ws_bytes < layer_ws(D, w->hidden, n_q, &oq, &ok, &ov, &oa, &ox, &op, &pf)) return TQ_HIP_EINVAL;
     unsigned char *ws = (unsigned char *)d_ws;
     float *q = (float *)(ws + oq), *k = (float *)(ws + ok), *v = (float *)(ws + ov);
     float *attn = (float *)(ws + oa);
@@ -1211,9 +1209,7 @@ int tq_hip_attention_layer_batch_async(tq_hip_kv *kv, const tq_hip_attn_weights 
     if (pos0 < 0 || pos0 + n > capacity_of(kv, seq)) return TQ_HIP_EINVAL;
     const tq_hip_kv_desc &D = kv->desc;
     size_t oq, ok, ov, oa, ox, op, pf;
-    const size_t full = layer_ws(D, w->hidden, n, &oq, &ok, &ov, &oa, &ox, &op, &pf);
-    if (ws_bytes < (n < 16 ? op : full)) return TQ_HIP_EINVAL;
-    if (ws_bytes < full) pf = 0;   // 9-15 rows without room for partials: no K splits
+    if (ws_bytes < layer_ws(D, w->hidden, n, &oq, &ok, &ov, &oa, &ox, &op, &pf)) return TQ_HIP_EINVAL;
     unsigned char *ws = (unsigned char *)d_ws;
     float *q = (float *)(ws + oq), *k = (float *)(ws + ok), *v = (float *)(ws + ov);
     float *attn = (float *)(ws + oa);

@@ -301,6 +301,43 @@ def test_attention_layer_batch_of_sequences(nat, oracle):
     kv.close()
 
 
+def test_attention_layer_rows_up_to_15_are_the_row_alone(nat):
+    """12 sequences' next tokens in one call and one by one: the same K and V
+    rows in the cache, codes and scales, at a shape where splitting K over
+    q/k/v would be the faster from 9 rows on."""
+    lib = nat.load()
+    nq, nkv, hd, hidden, n, pos = 32, 8, 128, 8192, 12, 3
+    rng = np.random.default_rng(1)
+    dims = ((nq * hd, hidden), (nkv * hd, hidden), (nkv * hd, hidden), (hidden, nq * hd))
+    mats = []
+    for r, c in dims:
+        m = blocks(r * c // QK)
+        m["d"] = rng.uniform(0.5, 1.5, m.size).astype(np.float32) * 0.0003
+        m["q"] = rng.integers(-127, 128, m["q"].shape, np.int8)
+        mats.append(m)
+    norm = np.ones(hd, np.float32)
+    L = DeviceLayer(nat, (*mats, norm, norm), dims, hidden, 1e-6)
+    x = normal(n * hidden, 2)
+    seen = []
+    for calls in ([list(range(n))], [[i] for i in range(n)]):
+        kv = nat.PagedKV(nq, nkv, hd, n_pages=n, max_seqs=n, max_pages_per_seq=1)
+        for i in range(n):
+            kv.set_pages(i, [i])
+        for seqs in calls:
+            rows = len(seqs)
+            wsb = lib.tq_hip_attention_layer_ws_bytes(kv.h, C_ref(L.w), rows)
+            ws, dout = nat.DeviceBuffer(wsb), nat.DeviceBuffer(rows * hidden * 4)
+            bufs = [dev(nat, np.array(seqs, np.int32)), dev(nat, np.full(rows, pos, np.int32)),
+                    dev(nat, x.reshape(n, hidden)[seqs])]
+            nat.check(lib.tq_hip_attention_layer_async(kv.h, C_ref(L.w), rows, bufs[0].ptr, bufs[1].ptr, pos,
+                                                       bufs[2].ptr, None, None, dout.ptr, ws.ptr, wsb, None), "layer")
+            nat.check(lib.tq_hip_stream_synchronize(kv.stream), "sync")
+        seen.append(np.stack([np.frombuffer(part.tobytes(), np.int32) for i in range(n) for part in kv.read(i, pos, 1)]))
+        kv.close()
+    assert seen[0].any(axis=1).all()
+    assert np.array_equal(seen[0], seen[1])
+
+
 def test_attention_layer_errors(nat, oracle):
     lib = nat.load()
     from tailorquantkernel_amd import native
