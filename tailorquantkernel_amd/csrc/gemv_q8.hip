@@ -514,6 +514,10 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
     static_assert(!XS || UNI, "the split layout is copied from uniform bases");
     using G = GemmTile<TT>;
     constexpr int T2 = G::T2;
+    // two blocks' weight scales at a time where all four do not fit the
+    // registers (128-token Q4 tiles of block_q8 rows spilled 5: 28,672 x 4,096
+    // over 2,048 tokens 698 us, now 640)
+    constexpr bool kScaleEach = Q4 && UNI && !XS && TT == 128;
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -700,24 +704,28 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         }
     };
 
-    // kGemmCopies direct-to-LDS copies per thread per stage, nothing else
+    // The same from per-lane addresses; LDS addresses from the wave's number, in
+    // scalar registers (from tid - lane they are vector ones, and the 128-token
+    // Q8 tile spilled 12 of them: rows of 4,032 / 960 / 960 x 4,096 over 2,048
+    // tokens 180 us, now 154)
+    const int tid0 = 64 * wave;
     auto issue = [&](int st, unsigned char *buf) {
         const int b0 = st * kGemmKB;
         const int bw = b0 + my_blk < nb ? b0 + my_blk : nb - 1;
         if (Q4) {
-            dma16(wrow + 16 * bw, buf + 16 * (tid - lane));
+            dma16(wrow + 16 * bw, buf + 16 * tid0);
         } else {
 #pragma unroll
             for (int half = 0; half < 2; half++)
-                dma16(wrow + tiled_offset(nb, bw, 16 * half), buf + 16 * (tid - lane + kGemmThreads * half));
+                dma16(wrow + tiled_offset(nb, bw, 16 * half), buf + 16 * (tid0 + kGemmThreads * half));
         }
-        dma4(drow + (b0 + (tid & 3) < nb ? b0 + (tid & 3) : nb - 1), buf + kGemmA + 4 * (tid - lane));
+        dma4(drow + (b0 + (tid & 3) < nb ? b0 + (tid & 3) : nb - 1), buf + kGemmA + 4 * tid0);
         if (BX4) {
             // the last round's copies past the tile are left out (whole waves)
 #pragma unroll
             for (int j = 0; j < G::ROUNDS; j++)
                 if (tid + kGemmThreads * j < G::CHUNKS)
-                    dma16(bsrc[j] + b0 * kBlockBytes, buf + kGemmA + kGemmWD + 16 * (tid + kGemmThreads * j - lane));
+                    dma16(bsrc[j] + b0 * kBlockBytes, buf + kGemmA + kGemmWD + 16 * (tid0 + kGemmThreads * j));
         } else {
 #pragma unroll
             for (int j = 0; j < (G::WORDS + kGemmThreads - 1) / kGemmThreads; j++) {
@@ -728,7 +736,7 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
                 const int t = tok0 + tk < a.n_tok ? tok0 + tk : a.n_tok - 1;
                 const int b = b0 + blk < nb ? b0 + blk : nb - 1;
                 dma4(a.xq + ((size_t)t * nb + b) * kBlockBytes + 4 * (w - 9 * blk),
-                     buf + kGemmA + kGemmWD + 4 * (c - lane));
+                     buf + kGemmA + kGemmWD + 4 * (tid0 + kGemmThreads * j));
             }
         }
     };
@@ -758,12 +766,14 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
         }
         const unsigned char *A = buf, *WD = buf + kGemmA, *B = buf + kGemmA + kGemmWD;
         // the row's four scales (times 1/16 for the Q4 codes, which come as 16 x code)
-        float4 wd4 = *reinterpret_cast<const float4 *>(WD + (wr + l32) * 16);
+        float4 wd4 = float4{};
+        if (!kScaleEach) wd4 = *reinterpret_cast<const float4 *>(WD + (wr + l32) * 16);
         if (Q4) wd4 = make_float4(wd4.x * 0.0625f, wd4.y * 0.0625f, wd4.z * 0.0625f, wd4.w * 0.0625f);
 #pragma unroll
         for (int b2 = 0; b2 < kGemmKB; b2 += 2) {
             // both blocks' scales: lane (l32, hi) holds those of block b2 + hi
-            const float wd = b2 == 0 ? (hi ? wd4.y : wd4.x) : (hi ? wd4.w : wd4.z);
+            float wd = b2 == 0 ? (hi ? wd4.y : wd4.x) : (hi ? wd4.w : wd4.z);
+            if (kScaleEach) wd = *reinterpret_cast<const float *>(WD + (wr + l32) * 16 + 4 * (b2 + hi)) * 0.0625f;
             float xd[T2];
 #pragma unroll
             for (int t2 = 0; t2 < T2; t2++) {

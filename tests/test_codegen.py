@@ -1,7 +1,7 @@
-"""The gfx950 code of the built library against the waits that the hardware
-does not make by itself and that the compiler does not add around inline
-assembly (its hazard pass takes an asm block as one instruction).  CPU only:
-llvm-objdump over the library built here from source."""
+"""The gfx950 code of the built library: the waits that the hardware does not
+make by itself and that the compiler does not add around inline assembly (its
+hazard pass takes an asm block as one instruction), and no register spilled to
+memory.  CPU only: ROCm's binary tools over the library built here from source."""
 from __future__ import annotations
 
 import glob
@@ -15,6 +15,9 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "tailorquantkernel_amd", "libtqhip.so")
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+needs_tools = pytest.mark.skipif(not (os.path.exists(OBJDUMP) and os.path.exists(READELF)),
+                                 reason="needs ROCm's llvm-objdump and llvm-readelf")
 
 
 def scalar_regs(text: str) -> set[str]:
@@ -60,12 +63,19 @@ def test_hazard_scan():
     assert hazards(["v_readfirstlane_b32 s6, v9", "s_mov_b32 m0, s6", "s_nop 0", load]) == (1, [])
 
 
-@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="needs ROCm's llvm-objdump")
-def test_copies_into_lds_wait_for_their_operands(tmp_path):
-    shutil.copy(LIB, tmp_path / "lib.so")
-    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+@pytest.fixture(scope="module")
+def objects(tmp_path_factory):
+    """The library's gfx950 code objects, one per source file."""
+    tmp = tmp_path_factory.mktemp("codegen")
+    shutil.copy(LIB, tmp / "lib.so")
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=tmp, check=True, stdout=subprocess.DEVNULL)
+    return sorted(glob.glob(str(tmp / "*gfx950")))
+
+
+@needs_tools
+def test_copies_into_lds_wait_for_their_operands(objects):
     copies, bad = 0, []
-    for obj in sorted(glob.glob(str(tmp_path / "*gfx950"))):
+    for obj in objects:
         asm = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", obj],
                              check=True, capture_output=True, text=True).stdout
         n, b = hazards(asm.splitlines())
@@ -73,3 +83,16 @@ def test_copies_into_lds_wait_for_their_operands(tmp_path):
         bad += b
     assert copies > 0, "no copy into LDS found: the scan no longer reads the code"
     assert not bad, f"{len(bad)} of {copies} copies, first: {bad[0]}"
+
+
+@needs_tools
+def test_no_kernel_spills(objects):
+    kernels, spilled = 0, []
+    for obj in objects:
+        notes = subprocess.run([READELF, "--notes", obj], check=True, capture_output=True, text=True).stdout
+        for name, n in re.findall(r"\.symbol: +(\S+?)\.kd.*?\.vgpr_spill_count: +(\d+)", notes, re.S):
+            kernels += 1
+            if int(n):
+                spilled.append((name, int(n)))
+    assert kernels > 100, "the kernels' notes are not read"
+    assert not spilled, spilled
