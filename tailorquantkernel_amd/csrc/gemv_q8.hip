@@ -1080,17 +1080,33 @@ bool gemm_uniform(const GemvArgs &a) {
     return (size_t)a.n_tok * a.nb * kBlockBytes < ((size_t)1 << 31);
 }
 
+// Work-groups of a launch without K splits (row tiles per XCD rounded up).
+long gemm_wgs(int rows, int n_tok, int toks) {
+    return ((long)(rows + kGemmRows - 1) / kGemmRows + 7) / 8 * 8 * ((n_tok + toks - 1) / toks);
+}
+
 // Tokens per tile of a launch over n_tok: 64 where one such tile holds them,
 // and up to 320 tokens where 128-token tiles would be half padding at the end
 // (an odd count of 64s; a 64-token tile takes 0.54 of a 128-token one).  8B
 // MLP, us with 64 / 128, Q8 then Q4: 130 tokens 140 / 155, 131 / 150; 190: 142
 // / 155, 135 / 154; 300: 206 / 225, 206 / 224.  At 420 the gain is gone (277 /
-// 282, 283 / 277) and at 550 it is a loss (371 / 345).  Attention layers: 8B,
-// 129 tokens 98 / 107, 320: 183 / 193; 70B, 320: 308 / 313, Q4 317 / 305 (its
-// 240 tiles of 128 split K in two, 400 of 64 do not: the one shape that lost).
+// 282, 283 / 277) and at 550 it is a loss (371 / 345).
+//
+// Five tiles of 64 against three of 128 lose where they alone give every CU a
+// work-group and so end the K splits (`split`: the launch may split) that three
+// leave room for: 7,169 to 10,240 rows.  MLP over 320 tokens, us with 64 / 128, Q8
+// then Q4: 8,192 x 28,672 809 / 789, 818 / 786; 7,168 x 4,096 135 / 133, 151 /
+// 136; 8,192 x 5,120 163 / 168, 175 / 171.  (Three of 64 against two do not
+// lose so: 4,096 x 7,168 over 160 tokens 80 / 86, 85 / 87.)
 constexpr int kGemmSmallToks = 320;
+constexpr int kSplitWgs = 512;
 
-int gemm_toks(int n_tok) { return n_tok <= 64 || (n_tok <= kGemmSmallToks && (n_tok + 63) / 64 % 2) ? 64 : 128; }
+int gemm_toks(int rows, int n_tok, bool split) {
+    if (n_tok <= 64) return 64;
+    if (n_tok > kGemmSmallToks || (n_tok + 63) / 64 % 2 == 0) return 128;
+    const bool ends_splits = gemm_wgs(rows, n_tok, 64) >= kSplitWgs / 2 && gemm_wgs(rows, n_tok, 128) < kSplitWgs / 2;
+    return split && n_tok > 192 && ends_splits ? 128 : 64;
+}
 
 template <int TT>
 hipError_t launch_gemm_t(const GemvArgs &u, bool bx4, unsigned grid, hipStream_t s) {
@@ -1136,11 +1152,8 @@ hipError_t launch_gemm_t(const GemvArgs &u, bool bx4, unsigned grid, hipStream_t
 }
 
 hipError_t launch_gemm(const GemvArgs &a, int ksplit, hipStream_t s) {
-    const int toks = gemm_toks(a.n_tok);
-    const int n_rt = (a.rows_total + kGemmRows - 1) / kGemmRows;
-    const int n_tt = (a.n_tok + toks - 1) / toks;
-    const long groups = ((long)n_rt + 7) / 8;   // row tiles per XCD, rounded up
-    const long grid = groups * 8 * n_tt * ksplit;
+    const int toks = gemm_toks(a.rows_total, a.n_tok, ksplit > 1);
+    const long grid = gemm_wgs(a.rows_total, a.n_tok, toks) * ksplit;
     if (grid > INT32_MAX) return hipErrorInvalidValue;
     const bool bx4 = (((uintptr_t)a.xq & 15) == 0) && a.nb % kGemmKB == 0;
     GemvArgs u = a;
@@ -1184,12 +1197,11 @@ hipError_t launch_gemm(const GemvArgs &a, int ksplit, hipStream_t s) {
 // 114 / 105, 164 / 157.  The least is 16 tokens, as without a workspace: up to
 // 15 a row's bits are the GEMV's whatever its batch.  (Splits from 9 tokens
 // took 72 / 59 for 100 / 76 us of GEMV launches there, with other bits.)
-constexpr int kSplitWgs = 512;
 constexpr int kSplitMinTokens = 16;
 
 int gemm_ksplit(int rows, int cols, int n_tok) {
     if (n_tok < kSplitMinTokens) return 1;
-    const long wgs = ((long)(rows + kGemmRows - 1) / kGemmRows + 7) / 8 * 8 * ((n_tok + gemm_toks(n_tok) - 1) / gemm_toks(n_tok));
+    const long wgs = gemm_wgs(rows, n_tok, gemm_toks(rows, n_tok, true));
     // once every CU holds a tile, splitting adds occupancy but not CUs, and
     // the partials' traffic outweighs it (4,096 x 14,336 at 1,024 tokens)
     if (wgs >= kSplitWgs / 2) return 1;
