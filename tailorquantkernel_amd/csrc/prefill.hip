@@ -67,6 +67,7 @@
 // head and keeps that head's tile image in its own L2.
 #include <algorithm>
 
+#include "prefill_runs.hpp"
 #include "tq_common.hpp"
 
 namespace {
@@ -77,7 +78,6 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 
-constexpr int kKT = 32;                  // keys per tile
 constexpr int kMaxPrefillKeys = 65536;   // keys [0, kend) the dense path serves
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.0f;            // log2 headroom before the running max moves
@@ -535,16 +535,6 @@ struct PrefillArgs {
     const unsigned char *img;
 };
 
-
-// Key tiles query block b reads: keys [0, pos0 + its last query + 1).
-__host__ __device__ inline int block_tiles(int pos0, int n, int qb, int b) {
-    const int last = (b + 1) * qb < n ? (b + 1) * qb : n;
-    return (pos0 + last + kKT - 1) / kKT;
-}
-
-// Runs a block of nt tiles is cut into.
-__host__ __device__ inline int block_runs(int nt, int chunk) { return chunk == 0 ? 1 : (nt + chunk - 1) / chunk; }
-
 // Per-row state of one wave's NJ row tiles over a run of key tiles: o and
 // lsum are taken against moff (mrow, or 0 before any key); mrow is the running
 // max; thr the largest score - moff a tile may hold without moving the max
@@ -856,19 +846,9 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_block_kernel(PrefillA
     __shared__ __attribute__((aligned(16))) unsigned char tiles[4][I::BYTES];
     static_assert(2 * 4 * 64 * (MT * 16 + 8) <= 4 * I::BYTES, "the halves' row tiles fit the tile buffers");
     const int kvh = (int)blockIdx.x % a.n_kv;
-    int blk = a.qblocks - 1, sp = (int)blockIdx.x / a.n_kv;
-    if (a.chunk == 0) {
-        blk -= sp;
-        sp = 0;
-    } else {
-        for (;; blk--) {
-            const int segs = block_runs(block_tiles(a.pos0, a.n, S::QB, blk), a.chunk);
-            if (sp < segs || blk == 0) break;
-            sp -= segs;
-        }
-    }
+    const BlockRun at_run = block_of_run(a.pos0, a.n, S::QB, a.qblocks, a.chunk, (int)blockIdx.x / a.n_kv);
+    const int blk = at_run.blk, sp = at_run.run, segs = at_run.runs;
     const int all = block_tiles(a.pos0, a.n, S::QB, blk);
-    const int segs = block_runs(all, a.chunk);
     // runs of whole tile pairs, as even as they go
     const int pairs = (all + 1) / 2;
     const int kt0 = 2 * (pairs * sp / segs);
@@ -1083,15 +1063,12 @@ PrefillPlan plan_prefill(int hd, int g, int n_kv_heads, int pos0, int n) {
     if (forced == 1 || (forced < 0 && (long)p.qblocks * n_kv_heads >= 2L * kCUs)) return p;
     const int most = block_tiles(pos0, n, qb, p.qblocks - 1);   // of the last, longest block
     const double unit = hd == 128 ? 1.0 : 1.5;                  // the fixed costs in steps, which are shorter at 64
+    long tiles = 0;
+    for (int b = 0; b < p.qblocks; b++) tiles += block_tiles(pos0, n, qb, b);
     double best = 0.0;
     for (int k = 1; k <= kMaxRuns && (k == 1 || (most + 1) / 2 >= k); k++) {
         const int chunk = (((most + k - 1) / k) + 1) & ~1;
-        long items = 0, tiles = 0;
-        for (int b = 0; b < p.qblocks; b++) {
-            const int nt = block_tiles(pos0, n, qb, b);
-            items += block_runs(nt, chunk);
-            tiles += nt;
-        }
+        const long items = total_runs(pos0, n, qb, p.qblocks, chunk);
         const int runs = block_runs(most, chunk);
         const double item = unit * (kItemCost + (runs > 1 ? kRunCost : 0.0));
         const double one = 0.5 * chunk + item + (runs > 1 ? unit * kMergeCost * runs : 0.0);
