@@ -81,11 +81,6 @@ typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 constexpr int kMaxPrefillKeys = 65536;   // keys [0, kend) the dense path serves
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.0f;            // log2 headroom before the running max moves
-constexpr int kMaxRuns = 8;              // runs of one query block
-// The plan's costs, in steps (a pair of key tiles, about 1.7 us at head_dim
-// 128): a work-group's prologue and store, its partial, and each run the last
-// one merges.
-constexpr double kItemCost = 3.5, kRunCost = 1.5, kMergeCost = 0.5;
 constexpr int kCounterStrideP = 64;      // ints: one 256-byte line per counter
 constexpr int kCoherentP = 16;           // cache policy sc1: agent-coherent access
 
@@ -1029,18 +1024,6 @@ int prefill_rows(int g) {
 // Query tokens per work-group for a shape (the kernel's QB).
 int prefill_qb(int g) { return 64 * (prefill_rows(g) == 128 ? 2 : 1) / g; }
 
-// With at least two query blocks per CU, every (query block, kv head) is one
-// work-group: dealt longest first, the blocks pair up on the CUs by
-// themselves.  With fewer, blocks may be cut into runs of `chunk` key tiles,
-// the length that minimises the modelled time: one work-group's (steps, fixed
-// cost, the merge of all runs by the last) while the launch is one round of
-// the CUs, else the CUs' share of all work plus half a work-group's.
-// Measured (us with 1, 2, 3, 4 and 8 runs of the longest block, 32 / 8 heads
-// of 128): 333 tokens after 1,000: 56.4 / 45.7 / 57.3 / 56.2 / 56.5; 100 after
-// 8,000: 255 / 149 / 112 / 95 / 74; 300 after none: 24.3 / 28.6 / 28.7 / - / -;
-// 1,024 after 1,024: 79.3 / 91 / 107 / 128 / 190; 8 / 2 heads of 64, 2,048
-// after none: 50 / 35 / 32 / 38 / 42.  The plan takes 2, 8, 1, 1 and 3.
-constexpr int kCUs = 256;                // compute units of an MI355X
 // TQ_HIP_PREFILL_WHOLE=1 keeps every block one run, =0 cuts every block into
 // as many runs as the plan may (tests of both at any size); read on every
 // call.  -1: the plan decides.
@@ -1052,36 +1035,10 @@ struct PrefillPlan {
     int qblocks, chunk, nsp, rows, items;
 };
 PrefillPlan plan_prefill(int hd, int g, int n_kv_heads, int pos0, int n) {
-    PrefillPlan p;
     const int qb = prefill_qb(g);
-    p.rows = 64 * (prefill_rows(g) == 128 ? 2 : 1);
-    p.qblocks = (n + qb - 1) / qb;
-    p.chunk = 0;
-    p.nsp = 1;
-    p.items = p.qblocks;
-    const int forced = prefill_whole_env();
-    if (forced == 1 || (forced < 0 && (long)p.qblocks * n_kv_heads >= 2L * kCUs)) return p;
-    const int most = block_tiles(pos0, n, qb, p.qblocks - 1);   // of the last, longest block
-    const double unit = hd == 128 ? 1.0 : 1.5;                  // the fixed costs in steps, which are shorter at 64
-    long tiles = 0;
-    for (int b = 0; b < p.qblocks; b++) tiles += block_tiles(pos0, n, qb, b);
-    double best = 0.0;
-    for (int k = 1; k <= kMaxRuns && (k == 1 || (most + 1) / 2 >= k); k++) {
-        const int chunk = (((most + k - 1) / k) + 1) & ~1;
-        const long items = total_runs(pos0, n, qb, p.qblocks, chunk);
-        const int runs = block_runs(most, chunk);
-        const double item = unit * (kItemCost + (runs > 1 ? kRunCost : 0.0));
-        const double one = 0.5 * chunk + item + (runs > 1 ? unit * kMergeCost * runs : 0.0);
-        const double work = n_kv_heads * (0.5 * tiles + items * item) / kCUs;
-        const double cost = items * n_kv_heads <= kCUs ? one : std::max(one, work + 0.5 * one);
-        if (forced == 0 || k == 1 || cost < best) {
-            best = cost;
-            p.chunk = k == 1 ? 0 : chunk;
-            p.nsp = runs;
-            p.items = (int)items;
-        }
-    }
-    return p;
+    const int qblocks = (n + qb - 1) / qb;
+    const RunPlan r = plan_runs(hd, qb, n_kv_heads, pos0, n, qblocks, prefill_whole_env());
+    return PrefillPlan{qblocks, r.chunk, r.runs, 64 * (prefill_rows(g) == 128 ? 2 : 1), r.items};
 }
 
 // Byte offset of the staged q blocks in the image buffer (after the key

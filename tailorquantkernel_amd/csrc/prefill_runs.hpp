@@ -3,6 +3,9 @@
 // use the same functions.
 #pragma once
 
+#include <algorithm>
+#include <cmath>
+
 namespace tq {
 
 constexpr int kKT = 32;   // keys per tile
@@ -57,6 +60,72 @@ __host__ __device__ inline long total_runs(int pos0, int n, int qb, int qblocks,
         hi = lo - 1;
     }
     return sum;
+}
+
+// How the blocks are cut: key tiles per run (0: every block is one run), the
+// longest block's runs, runs of all blocks.
+struct RunPlan {
+    int chunk, runs, items;
+};
+
+constexpr int kCUs = 256;       // compute units of an MI355X
+constexpr int kMaxRuns = 8;     // runs of one query block
+// The plan's costs, in steps (a pair of key tiles, about 1.7 us at head_dim
+// 128): a work-group's prologue and store, its partial, and each run the last
+// one merges.
+constexpr double kItemCost = 3.5, kRunCost = 1.5, kMergeCost = 1.0;
+
+// With at least two query blocks per CU, every (query block, kv head) is one
+// work-group: dealt longest first, the blocks pair up on the CUs by
+// themselves.  With fewer, blocks may be cut into runs of `chunk` key tiles,
+// the length that minimises the modelled time.  While the launch is one round
+// of the CUs that is one work-group's (steps, fixed cost).  Whole blocks of
+// head_dim 128 in more than one round are exactly predictable: a CU holds one
+// work-group, so the shortest of the first round frees the first CU, and block
+// 257 of the order pairs with 256, 258 with 255, ...  Otherwise it is the CUs'
+// share of all work, rounds taken halfway to whole ones, and a third of a
+// work-group's at the end.  The merge of all runs by the last comes on top.
+//
+// Over 100 measured shapes with fewer than 512 blocks or little above, each with
+// 1 to 8 runs, the plan's choice takes 1.0 % longer than the best of the eight in
+// the mean, 15 % at most.  Choices, us of the choice and the next best: 32 / 8
+// heads of 128, 2,000 after 2,000: whole 227, two runs 277; 333 after 1,000: two
+// 46, whole 56; 100 after 8,000: eight 74, four 95; 16 / 4, 4,000 after none: whole
+// 155, two 195; 8 / 2 of 64, 4,000 after 4,000: two 141, whole 174; 2,048 after
+// none: three 32, two 35.
+//
+// forced: 1 keeps every block one run, 0 cuts every block into as many runs as
+// may be, -1 lets the costs decide.
+inline RunPlan plan_runs(int hd, int qb, int n_kv_heads, int pos0, int n, int qblocks, int forced) {
+    RunPlan p{0, 1, qblocks};
+    if (forced == 1 || (forced < 0 && (long)qblocks * n_kv_heads >= 2L * kCUs)) return p;
+    const int most = block_tiles(pos0, n, qb, qblocks - 1);   // of the last, longest block
+    // time of the i-th longest (block, kv head) as one work-group
+    auto whole = [&](int i) { return 0.5 * block_tiles(pos0, n, qb, qblocks - 1 - i / n_kv_heads) + kItemCost; };
+    long tiles = 0;
+    for (int b = 0; b < qblocks; b++) tiles += block_tiles(pos0, n, qb, b);
+    double best = 0.0;
+    for (int k = 1; k <= kMaxRuns && (k == 1 || (most + 1) / 2 >= k); k++) {
+        const int chunk = (((most + k - 1) / k) + 1) & ~1;
+        const long items = total_runs(pos0, n, qb, qblocks, chunk), wgs = items * n_kv_heads;
+        const int runs = block_runs(most, chunk);
+        const double item = kItemCost + (runs > 1 ? kRunCost : 0.0), one = 0.5 * (k == 1 ? most : chunk) + item;
+        double cost;
+        if (wgs <= kCUs) {
+            cost = one;
+        } else if (k == 1 && hd == 128 && wgs < 2 * kCUs) {
+            cost = std::max({one, whole(kCUs - 1) + whole(kCUs), whole(2 * kCUs - 1 - (int)wgs) + whole((int)wgs - 1)});
+        } else {
+            const double rounds = (double)wgs / kCUs, share = n_kv_heads * (0.5 * tiles + items * item) / kCUs;
+            cost = std::max(one, share * 0.5 * (1.0 + std::ceil(rounds) / rounds) + 0.3 * one);
+        }
+        if (runs > 1) cost += kMergeCost * runs;
+        if (forced == 0 || k == 1 || cost < best) {
+            best = cost;
+            p = RunPlan{k == 1 ? 0 : chunk, runs, (int)items};
+        }
+    }
+    return p;
 }
 
 }  // namespace tq

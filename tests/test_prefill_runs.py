@@ -1,5 +1,6 @@
 """The prefill's (block, run) lookup against the count it replaces, block by
-block, over the sizes and cuts the plan can make; CPU only."""
+block, over the sizes and cuts the plan can make, and the cuts the plan takes
+where they were measured; CPU only."""
 from __future__ import annotations
 
 import os
@@ -39,11 +40,45 @@ int main() {
 """
 
 
-@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
-def test_block_of_run_equals_the_count(tmp_path):
-    src, exe = tmp_path / "runs.cpp", tmp_path / "runs"
-    src.write_text(HARNESS)
+PLAN = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "prefill_runs.hpp"
+int main(int, char **v) {
+    const int nq = atoi(v[1]), nkv = atoi(v[2]), hd = atoi(v[3]), n = atoi(v[4]), pos0 = atoi(v[5]), qb = 128 / (nq / nkv);
+    std::printf("%d\n", tq::plan_runs(hd, qb, nkv, pos0, n, (n + qb - 1) / qb, -1).runs);
+}
+"""
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+
+
+def build(tmp, text):
+    src, exe = tmp / "runs.cpp", tmp / "runs"
+    src.write_text(text)
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-D__host__=", "-D__device__=",
                     "-I", os.path.join(ROOT, "tailorquantkernel_amd", "csrc"), "-o", str(exe), str(src)], check=True)
-    seen, wrong = map(int, subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split())
+    return lambda *args: subprocess.run([str(exe), *map(str, args)], check=True, capture_output=True, text=True).stdout.split()
+
+
+def test_block_of_run_equals_the_count(tmp_path):
+    seen, wrong = map(int, build(tmp_path, HARNESS)())
     assert seen > 100_000 and wrong == 0, (seen, wrong)
+
+
+def test_plan_takes_the_measured_cuts(tmp_path):
+    """Whole blocks in more than one round of the CUs where those were the
+    fastest of 1 to 8 runs (the times beside each), runs where runs were."""
+    plan = build(tmp_path, PLAN)
+    for shape, runs in (((32, 8, 128, 2000, 2000), 1),     # us whole 227, two runs 277
+                        ((32, 8, 128, 2000, 8000), 1),     # 597, 627
+                        ((16, 4, 128, 4000, 0), 1),        # 155, 195
+                        ((16, 2, 128, 4000, 0), 1),        # 151, 192
+                        ((64, 8, 128, 1000, 16000), 1),    # 1059, 1111
+                        ((8, 1, 128, 8000, 0), 1),         # 275, 336
+                        ((8, 2, 64, 4000, 4000), 2),       # two runs 141, whole 174
+                        ((16, 4, 128, 2048, 0), 3),        # three 73, whole 77
+                        ((32, 8, 128, 333, 1000), 2),
+                        ((32, 8, 128, 100, 8000), 8),
+                        ((8, 2, 64, 2048, 0), 3)):
+        assert plan(*shape) == [str(runs)], shape
