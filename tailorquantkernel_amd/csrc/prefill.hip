@@ -516,7 +516,8 @@ struct PrefillArgs {
     int pos0;
     int n;
     int qblocks;         // query blocks of QB tokens
-    int chunk;           // key tiles per run of a block (0: every block is one run)
+    int whole;           // longest blocks of one run each
+    int chunk;           // key tiles per run of the others (0: one run too)
     int nsp;             // most runs of one block
     int n_kv;
     float *partials;     // [n_kv][qblocks][nsp][RW][HD + 4]
@@ -841,7 +842,7 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_block_kernel(PrefillA
     __shared__ __attribute__((aligned(16))) unsigned char tiles[4][I::BYTES];
     static_assert(2 * 4 * 64 * (MT * 16 + 8) <= 4 * I::BYTES, "the halves' row tiles fit the tile buffers");
     const int kvh = (int)blockIdx.x % a.n_kv;
-    const BlockRun at_run = block_of_run(a.pos0, a.n, S::QB, a.qblocks, a.chunk, (int)blockIdx.x / a.n_kv);
+    const BlockRun at_run = plan_item(a.pos0, a.n, S::QB, a.qblocks, a.whole, a.chunk, (int)blockIdx.x / a.n_kv);
     const int blk = at_run.blk, sp = at_run.run, segs = at_run.runs;
     const int all = block_tiles(a.pos0, a.n, S::QB, blk);
     // runs of whole tile pairs, as even as they go
@@ -1032,13 +1033,13 @@ int prefill_whole_env() {
     return (s && *s) ? (s[0] == '1' ? 1 : 0) : -1;
 }
 struct PrefillPlan {
-    int qblocks, chunk, nsp, rows, items;
+    int qblocks, whole, chunk, nsp, rows, items;
 };
 PrefillPlan plan_prefill(int hd, int g, int n_kv_heads, int pos0, int n) {
     const int qb = prefill_qb(g);
     const int qblocks = (n + qb - 1) / qb;
     const RunPlan r = plan_runs(hd, qb, n_kv_heads, pos0, n, qblocks, prefill_whole_env());
-    return PrefillPlan{qblocks, r.chunk, r.runs, 64 * (prefill_rows(g) == 128 ? 2 : 1), r.items};
+    return PrefillPlan{qblocks, r.whole, r.chunk, r.runs, 64 * (prefill_rows(g) == 128 ? 2 : 1), r.items};
 }
 
 // Byte offset of the staged q blocks in the image buffer (after the key
@@ -1134,6 +1135,7 @@ hipError_t tq_launch_prefill(const TqPrefillArgs &t, hipStream_t s) {
     a.qimg = t.img + qimg_offset(t.head_dim, t.n_kv_heads, t.pos0 + t.n);
     const PrefillPlan p = plan_prefill(t.head_dim, g, t.n_kv_heads, t.pos0, t.n);
     a.qblocks = p.qblocks;
+    a.whole = p.whole;
     a.chunk = p.chunk;
     a.nsp = p.nsp;
     a.n_kv = t.n_kv_heads;

@@ -62,11 +62,19 @@ __host__ __device__ inline long total_runs(int pos0, int n, int qb, int qblocks,
     return sum;
 }
 
-// How the blocks are cut: key tiles per run (0: every block is one run), the
-// longest block's runs, runs of all blocks.
+// How the blocks are cut: the `whole` longest are one run each, the others have
+// runs of at most `chunk` key tiles (0: one run); `runs` is the most of a block,
+// `items` all of them.
 struct RunPlan {
-    int chunk, runs, items;
+    int whole, chunk, runs, items;
 };
+
+// Item `item` of a plan.
+__host__ __device__ inline BlockRun plan_item(int pos0, int n, int qb, int qblocks, int whole, int chunk, int item) {
+    if (item < whole) return BlockRun{qblocks - 1 - item, 0, 1};
+    const int cut = qblocks - whole;
+    return block_of_run(pos0, whole > 0 ? cut * qb : n, qb, cut, chunk, item - whole);
+}
 
 constexpr int kCUs = 256;       // compute units of an MI355X
 constexpr int kMaxRuns = 8;     // runs of one query block
@@ -86,9 +94,16 @@ constexpr double kItemCost = 3.5, kRunCost = 1.5, kMergeCost = 1.0;
 // share of all work, rounds taken halfway to whole ones, and a third of a
 // work-group's at the end.  The merge of all runs by the last comes on top.
 //
-// Over 100 measured shapes with fewer than 512 blocks or little above, each with
-// 1 to 8 runs, the plan's choice takes 1.0 % longer than the best of the eight in
-// the mean, 15 % at most.  Choices, us of the choice and the next best: 32 / 8
+// A little over one round of equal blocks (keys before the prompt) suits no
+// such cut: whole, the second round is nearly empty, and in runs of all blocks
+// every one pays for the cut.  There the longest blocks that fill the CUs once stay
+// whole and only the others are cut, to run on the CUs left and then beside
+// them: share of all work and half a run at the end.  32 / 8 heads of 128, us so,
+// whole and in three runs: 1,100 after 2,000 129, 161, 166; after 8,000 346, 511,
+// 400; 64 / 8, 600 after 4,000 201, 274, 236.
+//
+// Over 100 measured shapes, each with its blocks in 1 to 8 runs, the choice among
+// those eight takes 1.0 % longer than the best in the mean, 15 % at most.  Choices, us of the choice and the next best: 32 / 8
 // heads of 128, 2,000 after 2,000: whole 227, two runs 277; 333 after 1,000: two
 // 46, whole 56; 100 after 8,000: eight 74, four 95; 16 / 4, 4,000 after none: whole
 // 155, two 195; 8 / 2 of 64, 4,000 after 4,000: two 141, whole 174; 2,048 after
@@ -97,7 +112,7 @@ constexpr double kItemCost = 3.5, kRunCost = 1.5, kMergeCost = 1.0;
 // forced: 1 keeps every block one run, 0 cuts every block into as many runs as
 // may be, -1 lets the costs decide.
 inline RunPlan plan_runs(int hd, int qb, int n_kv_heads, int pos0, int n, int qblocks, int forced) {
-    RunPlan p{0, 1, qblocks};
+    RunPlan p{0, 0, 1, qblocks};
     if (forced == 1 || (forced < 0 && (long)qblocks * n_kv_heads >= 2L * kCUs)) return p;
     const int most = block_tiles(pos0, n, qb, qblocks - 1);   // of the last, longest block
     // time of the i-th longest (block, kv head) as one work-group
@@ -122,7 +137,21 @@ inline RunPlan plan_runs(int hd, int qb, int n_kv_heads, int pos0, int n, int qb
         if (runs > 1) cost += kMergeCost * runs;
         if (forced == 0 || k == 1 || cost < best) {
             best = cost;
-            p = RunPlan{k == 1 ? 0 : chunk, runs, (int)items};
+            p = RunPlan{0, k == 1 ? 0 : chunk, runs, (int)items};
+        }
+    }
+    const int full = kCUs / n_kv_heads, cut = qblocks - full;   // blocks of one round, and those beyond it
+    if (forced == 0 || hd != 128 || full < 1 || cut < 1 || qblocks * n_kv_heads <= kCUs) return p;
+    const int longest = block_tiles(pos0, n, qb, cut - 1);
+    for (int k = 2; k <= kMaxRuns && (longest + 1) / 2 >= k; k++) {
+        const int chunk = (((longest + k - 1) / k) + 1) & ~1;
+        const long items = total_runs(pos0, cut * qb, qb, cut, chunk);
+        const double run = kItemCost + kRunCost, share = n_kv_heads * (0.5 * tiles + full * kItemCost + items * run) / kCUs;
+        const int runs = block_runs(longest, chunk);
+        const double cost = std::max(0.5 * most + kItemCost, share + 0.5 * (0.5 * chunk + run)) + kMergeCost * runs;
+        if (cost < best) {
+            best = cost;
+            p = RunPlan{full, chunk, runs, full + (int)items};
         }
     }
     return p;

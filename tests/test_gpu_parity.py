@@ -585,6 +585,34 @@ def test_prefill_runs(nat, oracle, nq, nkv, hd, pos0, n, monkeypatch):
     assert err.max() <= T * 2.0 ** -22 * np.abs(outs[1]).max(), err.max()
 
 
+@pytest.mark.parametrize("nq,nkv,n,pos0", [(64, 64, 600, 700), (128, 32, 280, 700), (256, 32, 131, 600)])
+def test_prefill_cuts_the_blocks_past_one_round(nat, oracle, nq, nkv, n, pos0, monkeypatch):
+    """A little over one query block per CU: the plan keeps the longest blocks
+    whole (the same bits as with every block whole) and cuts the others, here
+    the first (other bits, the bound of test_prefill_runs)."""
+    hd, T, block = 128, pos0 + n, 128 * nkv // nq
+    q, k, v = (normal(n * h * hd, 50 + i) for i, h in enumerate((nq, nkv, nkv)))
+    pre = [oracle.quantize_row_q8(normal(nkv * T * hd, 60 + i)).reshape(nkv, T, hd // QK) for i in range(2)]
+    outs = []
+    for env in (None, "1", None):
+        if env:
+            monkeypatch.setenv("TQ_HIP_PREFILL_WHOLE", env)
+        else:
+            monkeypatch.delenv("TQ_HIP_PREFILL_WHOLE", raising=False)
+        kv = nat.PagedKV.single(nq, nkv, hd, T)
+        kv.write(0, 0, *pre)
+        rc, out = kv.prefill(0, pos0, n, q, k, v)
+        assert rc == 0
+        outs.append(out)
+        kv.close()
+    bits = [o.view(np.int32) for o in outs]
+    assert np.array_equal(bits[0], bits[2])
+    assert np.array_equal(bits[0][block:], bits[1][block:])
+    assert not np.array_equal(bits[0][:block], bits[1][:block])
+    err = np.abs(outs[0].astype(np.float64) - outs[1])
+    assert err.max() <= T * 2.0 ** -22 * np.abs(outs[1]).max(), err.max()
+
+
 def check_prefill(nat, oracle, shape):
     nq, nkv, hd, T, theta, pos0, n = shape
     nb = hd // QK

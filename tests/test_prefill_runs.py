@@ -17,7 +17,7 @@ HARNESS = r"""
 #include "prefill_runs.hpp"
 using namespace tq;
 int main() {
-    long seen = 0, wrong = 0;
+    long seen = 0, wrong = 0, mixed = 0;
     for (int qb : {16, 32, 64, 128})
         for (int pos0 : {0, 1, 31, 32, 97, 1000, 4095, 8000, 65000})
             for (int n : {1, 15, 16, 17, 32, 33, 100, 127, 128, 129, 333, 2048, 4097, 8176})
@@ -35,7 +35,27 @@ int main() {
                     }
                     wrong += total_runs(pos0, n, qb, qblocks, chunk) != item;
                 }
-    std::printf("%ld %ld\n", seen, wrong);
+    // the plans themselves: every run once, whole blocks first, all counted
+    for (int nkv : {1, 2, 4, 8, 16, 32, 64, 100, 300})
+        for (int qb : {16, 32, 64, 128})
+            for (int pos0 : {0, 500, 2000, 4000, 8000, 30000})
+                for (int n = 1; n < 4300; n += n < 200 ? 13 : 101) {
+                    const int qblocks = (n + qb - 1) / qb;
+                    const RunPlan p = plan_runs(128, qb, nkv, pos0, n, qblocks, -1);
+                    mixed += p.whole > 0;
+                    int item = 0, most = 1;
+                    for (int b = qblocks - 1; b >= 0; b--) {
+                        const int cut = qblocks - 1 - b < p.whole ? 0 : p.chunk;
+                        const int runs = block_runs(block_tiles(pos0, n, qb, b), cut);
+                        most = runs > most ? runs : most;
+                        for (int s = 0; s < runs; s++, item++) {
+                            const BlockRun r = plan_item(pos0, n, qb, qblocks, p.whole, p.chunk, item);
+                            wrong += r.blk != b || r.run != s || r.runs != runs;
+                        }
+                    }
+                    wrong += item != p.items || most != p.runs || p.runs > kMaxRuns;
+                }
+    std::printf("%ld %ld %ld\n", seen, wrong, mixed);
 }
 """
 
@@ -46,7 +66,8 @@ PLAN = r"""
 #include "prefill_runs.hpp"
 int main(int, char **v) {
     const int nq = atoi(v[1]), nkv = atoi(v[2]), hd = atoi(v[3]), n = atoi(v[4]), pos0 = atoi(v[5]), qb = 128 / (nq / nkv);
-    std::printf("%d\n", tq::plan_runs(hd, qb, nkv, pos0, n, (n + qb - 1) / qb, -1).runs);
+    const tq::RunPlan p = tq::plan_runs(hd, qb, nkv, pos0, n, (n + qb - 1) / qb, -1);
+    std::printf("%d %d\n", p.whole, p.runs);
 }
 """
 
@@ -62,8 +83,8 @@ def build(tmp, text):
 
 
 def test_block_of_run_equals_the_count(tmp_path):
-    seen, wrong = map(int, build(tmp_path, HARNESS)())
-    assert seen > 100_000 and wrong == 0, (seen, wrong)
+    seen, wrong, mixed = map(int, build(tmp_path, HARNESS)())
+    assert seen > 100_000 and mixed > 100 and wrong == 0, (seen, wrong, mixed)
 
 
 def test_plan_takes_the_measured_cuts(tmp_path):
@@ -81,4 +102,7 @@ def test_plan_takes_the_measured_cuts(tmp_path):
                         ((32, 8, 128, 333, 1000), 2),
                         ((32, 8, 128, 100, 8000), 8),
                         ((8, 2, 64, 2048, 0), 3)):
-        assert plan(*shape) == [str(runs)], shape
+        assert plan(*shape) == ["0", str(runs)], shape
+    # a little over one round: 32 of 35 blocks whole, the others in runs
+    assert plan(32, 8, 128, 1100, 2000) == ["32", "3"]
+    assert plan(64, 8, 128, 600, 4000) == ["32", "4"]
