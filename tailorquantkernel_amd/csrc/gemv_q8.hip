@@ -1046,9 +1046,12 @@ hipError_t launch_gemv(const GemvArgs &a, int tcap, bool xf, int rw, int gc, hip
 }
 
 // One GEMV launch of up to tmax tokens streams the weights once, at about
-// 5 TB/s of Q8 bytes (Q4 launches of 8 tokens take as long: their vector work
-// is the same), plus its launch.
-double gemv_us(int rows, int cols) { return (double)rows * cols * (kBlockBytes / (double)kQK) / 5.0e6 + 2.5; }
+// 5 TB/s of Q8 bytes, plus its launch.  Q4 launches of 8 tokens take as long:
+// their vector work is the same.  Where 8 tokens do not fit, launches of 4 are
+// bound by their own bytes: 4,096 x 14,336 14.4 us, Q4 10.2.
+double gemv_us(int rows, int cols, bool q4, int tmax) {
+    return (double)rows * cols * (kBlockBytes / (double)kQK) / 5.0e6 * (tmax >= 8 ? 1.0 : q4 ? 0.6 : 0.9) + 2.5;
+}
 
 // From how many tokens on (block_q8 input) the unsplit MFMA GEMM runs instead
 // of GEMV launches of tmax tokens each (TQ_HIP_GEMM_MIN_TOKENS overrides).
@@ -1058,11 +1061,12 @@ double gemv_us(int rows, int cols) { return (double)rows * cols * (kBlockBytes /
 //   6144 x 4096    16 tokens 33 / 18    32: 33 / 33    64: 34 / 63    96: 58 / 94
 //   28672 x 4096    8: 48 / 35    12: 48 / 55    32: 48 / 121    96: 68 / 346
 //   4096 x 14336   16: 105 / 58   32: 105 / 116  64: 106 / 231   96: 190 / 345
-// The model puts the crossovers at 33, 16 (the least) and 28.
-int gemm_min_tokens(int rows, int cols, int tmax) {
+//   the same, Q4   28: 114 / 75   40: 114 / 106  48: 114 / 126   64: 114 / 164
+// The model puts the crossovers at 33, 16 (the least), 30 and 42.
+int gemm_min_tokens(int rows, int cols, bool q4, int tmax) {
     const int v = env_int("TQ_HIP_GEMM_MIN_TOKENS", 0);
     if (v > 0) return v;
-    const double per_token = gemv_us(rows, cols) / tmax;
+    const double per_token = gemv_us(rows, cols, q4, tmax) / tmax;
     const int n64 = (int)((0.0072 * cols + 3.5) / per_token) + 1;
     if (n64 <= 64) return n64 < 16 ? 16 : n64;   // up to 15 tokens a row's bits are the GEMV's whatever its batch
     const int n128 = (int)((0.0133 * cols + 3.5) / per_token) + 1;
@@ -1219,7 +1223,7 @@ int gemm_plan(const GemvArgs &a, int n_tok) {
     const int ksplit = a.part ? gemm_ksplit(a.rows_total, a.cols, n_tok) : 1;
     if (ksplit > 1 && (size_t)ksplit * n_tok * a.rows_total <= a.part_floats && env_int("TQ_HIP_GEMM_SPLIT", 1) != 0)
         return ksplit;
-    return n_tok >= gemm_min_tokens(a.rows_total, a.cols, pick_tokens(a.nb, false)) ? 1 : 0;
+    return n_tok >= gemm_min_tokens(a.rows_total, a.cols, a.q4, pick_tokens(a.nb, false)) ? 1 : 0;
 }
 
 // Whether the matmul's input should be quantized into the split layout:

@@ -15,7 +15,7 @@ import os
 import numpy as np
 import pytest
 
-from oracle.binding import QK, blocks4
+from oracle.binding import BLOCK_Q8, QK, blocks4
 from tests.golden.gen import fill_random
 
 pytestmark = pytest.mark.gpu
@@ -255,3 +255,26 @@ def test_q4_mlp_split_k(nat, oracle, split, monkeypatch):
     check_matmul(gate, oracle.matmul_q4(wg, xq, inter, hidden, n), wg, xq, inter, hidden, n, "gate")
     check_matmul(up, oracle.matmul_q4(wu, xq, inter, hidden, n), wu, xq, inter, hidden, n, "up")
     check_matmul(out, oracle.matmul_q4(wd, hq, hidden, inter, n), wd, hq, hidden, inter, n, "down")
+
+
+def test_q4_wide_rows_stay_with_gemv(nat, monkeypatch):
+    """14,336 columns: GEMV launches hold 4 tokens and a Q4 one takes 0.7 of a
+    Q8 one, so GEMV stays the default up to 40 tokens (its bits, those of the
+    forced route) and the GEMM takes 48."""
+    rows, cols = 4096, 14336
+    rng = np.random.default_rng(1)
+    Wq = blocks4(rows * cols // QK)
+    Wq["d"] = rng.uniform(0.5, 1.5, Wq.size).astype(np.float32) * 0.005
+    Wq["q"] = rng.integers(0, 256, Wq["q"].shape, np.uint8)
+    M = Matrix4(nat, Wq, rows, cols)
+    xq = np.zeros(48 * cols // QK, BLOCK_Q8)
+    xq["d"] = rng.uniform(0.5, 1.5, xq.size).astype(np.float32) * 0.01
+    xq["q"] = rng.integers(-127, 128, xq["q"].shape, np.int8)
+    for n, gemv in ((28, True), (40, True), (48, False)):
+        rows_n = xq[:n * cols // QK]
+        y = gpu_matmul4(nat, M, rows_n, n)
+        monkeypatch.setenv("TQ_HIP_GEMM_MIN_TOKENS", "1000")
+        forced = gpu_matmul4(nat, M, rows_n, n)
+        monkeypatch.delenv("TQ_HIP_GEMM_MIN_TOKENS")
+        assert np.array_equal(y.view(np.int32), forced.view(np.int32)) == gemv, n
+        assert rel_err(y, forced) <= 1e-5, n
