@@ -12,8 +12,8 @@
 //   contiguous tile image laid out as the MFMA operands want them (and, in
 //   the same launch, once per (query block, kv head): the block's q rows
 //   after RoPE, quantized exactly as quantize_row_q8 does, as int8 codes and
-//   fp32 scales in the layout prefill_kernel keeps them in LDS, so every
-//   segment of the block copies them instead of re-deriving them):
+//   fp32 scales in the layout the attention keeps them in LDS, so every run
+//   of the block copies them instead of re-deriving them):
 //     K codes [key half][block][lane][8 bf16]     (A of the score product)
 //     K scales [key half][block][lane group][4]   (kd of a lane's four keys)
 //     V' hi|lo [column tile][lane][8 bf16]        (A of the P.V product)
@@ -21,9 +21,9 @@
 //   fp32 and split into bf16 hi + lo (hi + lo = x to 2^-18 relative).  Every
 //   query block then streams these images instead of re-deriving them.
 //
-// The attention — per 4 waves, one kv head, 64*NJ
-//   (query, head) rows = QB = 64*NJ/G consecutive query tokens x the G heads
-//   of the group, in row tiles of 16 queries of one head; wave w owns NJ row
+// The attention — per 4 waves, one kv head, 128 (query, head) rows = QB =
+//   128/G consecutive query tokens x the G heads of the group, in row tiles
+//   of 16 queries of one head; wave w owns NJ = 2 row
 //   tiles.  The block's staged q codes go to registers as bf16 (exact), its
 //   scales times scale * log2(e) beside them.
 //   Key tiles are copied straight into two LDS buffers (global_load_lds), one
@@ -78,6 +78,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 
+constexpr int NJ = 2;                    // row tiles (of 16) per wave
 constexpr int kMaxPrefillKeys = 65536;   // keys [0, kend) the dense path serves
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.0f;            // log2 headroom before the running max moves
@@ -219,7 +220,7 @@ __device__ __forceinline__ v4f norm4(v4f x, float inv, v4f w) {
     return v4f{x.x * inv * w.x, x.y * inv * w.y, x.z * inv * w.z, x.w * inv * w.w};
 }
 
-template <int HD, int G, int NJ>
+template <int HD, int G>
 struct PShape {
     using I = TileImg<HD>;
     static constexpr int NB = I::NB;
@@ -239,9 +240,9 @@ struct PShape {
 // then scales [RW][NB].  Task (row r, c) covers q[4c..4c+3] and its
 // rotate-half partner q[HD/2+4c..+3]; every load of the thread's tasks is
 // issued before the first is used.  Rows of tokens past n are zero.
-template <int HD, int G, int NJ>
+template <int HD, int G>
 __device__ __forceinline__ void stage_q(const StageArgs &a, int kvh, int blk) {
-    using S = PShape<HD, G, NJ>;
+    using S = PShape<HD, G>;
     constexpr int NB = S::NB;
     constexpr int HALF = HD / 2;
     constexpr int CPR = HD / 8;                      // tasks per row; 8 | CPR
@@ -330,10 +331,10 @@ __device__ __forceinline__ void stage_q(const StageArgs &a, int kvh, int blk) {
 
 // Grid (n_tiles + qblocks, n_kv): x < n_tiles stages key tile x, the rest
 // stage q block x - n_tiles.
-template <int HD, int G, int NJ>
+template <int HD, int G>
 __global__ __launch_bounds__(kThreads) void prefill_stage_kernel(StageArgs a) {
     if ((int)blockIdx.x >= a.n_tiles) {
-        stage_q<HD, G, NJ>(a, blockIdx.y, (int)blockIdx.x - a.n_tiles);
+        stage_q<HD, G>(a, blockIdx.y, (int)blockIdx.x - a.n_tiles);
         return;
     }
     using I = TileImg<HD>;
@@ -537,9 +538,9 @@ struct PrefillArgs {
 // (kLazy; -inf before any key, so the first visible key takes the slow path);
 // lsum is this lane's share of the row sum, added over the row's lanes at the
 // end.  The same in the row's four lanes.
-template <int HD, int G, int NJ>
+template <int HD, int G>
 struct PRows {
-    static constexpr int MT = PShape<HD, G, NJ>::MT;
+    static constexpr int MT = PShape<HD, G>::MT;
     v4f o[MT][NJ];
     float mrow[NJ], moff[NJ], thr[NJ], lsum[NJ];
     __device__ __forceinline__ void init() {
@@ -560,19 +561,19 @@ struct PRows {
 // The score product's B operands of one wave's rows: the q codes of query
 // l16, values 32b + 8lg .. +7, as bf16 (exact), qd * scale * log2(e) per
 // block, and each row's query position.
-template <int HD, int G, int NJ>
+template <int HD, int G>
 struct PQ {
-    static constexpr int NB = PShape<HD, G, NJ>::NB;
+    static constexpr int NB = PShape<HD, G>::NB;
     v8bf qcb[NJ][NB];
     float qsc[NJ][NB];
     int qpos[NJ];
 };
 
 // From the block's staged q image in LDS (codes at qc, scales after them).
-template <int HD, int G, int NJ>
+template <int HD, int G>
 __device__ __forceinline__ void load_q(const PrefillArgs &a, const unsigned char *qc, int i0, int wave, int lane,
-                                       PQ<HD, G, NJ> &q) {
-    using S = PShape<HD, G, NJ>;
+                                       PQ<HD, G> &q) {
+    using S = PShape<HD, G>;
     constexpr int NB = S::NB;
     const int l16 = lane & 15, lg = lane >> 4;
     const float *qd = reinterpret_cast<const float *>(qc + S::RW * S::QCS);
@@ -597,7 +598,6 @@ __device__ __forceinline__ void load_q(const PrefillArgs &a, const unsigned char
 }
 
 // The P operands of one tile: P = exp2(S - moff) split into bf16 hi | lo.
-template <int NJ>
 struct PP {
     u32x4 hi[NJ], lo[NJ];
 };
@@ -605,10 +605,10 @@ struct PP {
 // One key tile kt (image T in LDS) against the wave's rows, first part:
 // exact scores, the causal mask, the online softmax (o and lsum rescaled when
 // the max moves) and this tile's P.
-template <int HD, int G, int NJ>
+template <int HD, int G>
 __device__ __forceinline__ void tile_scores(const PrefillArgs &a, const unsigned char *T, int kt, int i0, int lane,
-                                            const PQ<HD, G, NJ> &q, PRows<HD, G, NJ> &st, PP<NJ> &pp) {
-    using S = PShape<HD, G, NJ>;
+                                            const PQ<HD, G> &q, PRows<HD, G> &st, PP &pp) {
+    using S = PShape<HD, G>;
     using I = TileImg<HD>;
     constexpr int NB = S::NB;
     const int lg = lane >> 4;
@@ -704,9 +704,9 @@ __device__ __forceinline__ void tile_scores(const PrefillArgs &a, const unsigned
 }
 
 // Second part: O^T += V'^T . P^T with the tile's V' (image T) and its P.
-template <int HD, int G, int NJ>
-__device__ __forceinline__ void tile_pv(const unsigned char *T, int lane, const PP<NJ> &pp, PRows<HD, G, NJ> &st) {
-    using S = PShape<HD, G, NJ>;
+template <int HD, int G>
+__device__ __forceinline__ void tile_pv(const unsigned char *T, int lane, const PP &pp, PRows<HD, G> &st) {
+    using S = PShape<HD, G>;
     using I = TileImg<HD>;
 #pragma unroll
     for (int m = 0; m < S::MT; m++) {
@@ -722,21 +722,21 @@ __device__ __forceinline__ void tile_pv(const unsigned char *T, int lane, const 
 }
 
 // Both parts of one tile.
-template <int HD, int G, int NJ>
+template <int HD, int G>
 __device__ __forceinline__ void tile_update(const PrefillArgs &a, const unsigned char *T, int kt, int i0, int lane,
-                                            const PQ<HD, G, NJ> &q, PRows<HD, G, NJ> &st) {
-    PP<NJ> pp;
-    tile_scores<HD, G, NJ>(a, T, kt, i0, lane, q, st, pp);
-    tile_pv<HD, G, NJ>(T, lane, pp, st);
+                                            const PQ<HD, G> &q, PRows<HD, G> &st) {
+    PP pp;
+    tile_scores<HD, G>(a, T, kt, i0, lane, q, st, pp);
+    tile_pv<HD, G>(T, lane, pp, st);
 }
 
 // Normalise and store row tile nt (16 rows): lane holds columns
 // 16m + 4lg .. +3 of query l16.  Either fp32 rows into out, or (out_xs) each row quantized as
 // quantize_row_q8 straight into the split layout the output GEMM reads.
-template <int HD, int G, int NJ>
+template <int HD, int G>
 __device__ __forceinline__ void store_rows(const PrefillArgs &a, int kvh, int i0, int nt, int lane,
                                            const v4f (&o)[HD / 16], float lrow) {
-    using S = PShape<HD, G, NJ>;
+    using S = PShape<HD, G>;
     const int l16 = lane & 15, lg = lane >> 4;
     const float inv = 1.0f / lrow;
     const int g = nt / S::QT;
@@ -825,19 +825,19 @@ __device__ __forceinline__ bool tile_has_rem(int gwave) {
 // together (one barrier per pair of tiles, each half with its own two LDS
 // buffers, one tile ahead).  At the end each half hands one of its two row
 // tiles per wave to the other through LDS and merges its own with the one it
-// gets, in half order (NJ == 1: half 0 merges).
+// gets, in half order.
 //
 // A block covered by one run stores its rows.  With several, every work-group
 // writes its merged partial rows [RW][HD + 4] (o unnormalised, m, l) with
 // agent-coherent stores, waits for them, then arrives on the block's counter;
 // the last to arrive merges all of them in run order (its own from registers)
 // and puts the counter back to 0.  Nothing waits on another work-group.
-template <int HD, int G, int NJ>
+template <int HD, int G>
 __global__ __launch_bounds__(2 * kThreads, 1) void prefill_block_kernel(PrefillArgs a) {
-    using S = PShape<HD, G, NJ>;
+    using S = PShape<HD, G>;
     using I = TileImg<HD>;
     constexpr int MT = S::MT;
-    constexpr bool BOTH = NJ == 2;   // both halves finish a row tile per wave
+    static_assert(NJ == 2, "each half finishes one of its two row tiles per wave");
     // tile buffers: half 0 uses 0, 1; half 1 uses 2, 3
     __shared__ __attribute__((aligned(16))) unsigned char tiles[4][I::BYTES];
     static_assert(2 * 4 * 64 * (MT * 16 + 8) <= 4 * I::BYTES, "the halves' row tiles fit the tile buffers");
@@ -883,9 +883,9 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_block_kernel(PrefillA
     }
     __syncthreads();
 
-    PQ<HD, G, NJ> q;
-    load_q<HD, G, NJ>(a, tiles[1], i0, wave, lane, q);
-    PRows<HD, G, NJ> st;
+    PQ<HD, G> q;
+    load_q<HD, G>(a, tiles[1], i0, wave, lane, q);
+    PRows<HD, G> st;
     st.init();
 
     // Both halves step together, one barrier per step, each tile's scores
@@ -899,15 +899,15 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_block_kernel(PrefillA
         asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
         __syncthreads();
         if (s + 1 < mine) fetch_tile<HD>(img, 2 * (s + 1) + half, buf(s + 1), htid, wave);
-        if (s < mine) tile_update<HD, G, NJ>(a, buf(s), kt0 + 2 * s + half, i0, lane, q, st);
+        if (s < mine) tile_update<HD, G>(a, buf(s), kt0 + 2 * s + half, i0, lane, q, st);
     }
 
     float lrow[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) lrow[j] = xrow_sum(st.lsum[j]);
-    // row tile j of a half is finished by half j (BOTH) or half 0; the other
-    // half leaves it in the free tile buffers lane by lane (the waves of both
-    // halves hold the same rows and columns in the same lanes)
+    // row tile j of both halves is finished by half j; the other half leaves it
+    // in the free tile buffers lane by lane (the waves of both halves hold the
+    // same rows and columns in the same lanes)
     v4f *ob = reinterpret_cast<v4f *>(&tiles[0][0]);               // [from half][wave][MT][64]
     float *mb = reinterpret_cast<float *>(ob + 2 * 4 * MT * 64);   // [from half][wave][64] x (m, l)
     __syncthreads();   // every wave is done with the tile buffers
@@ -915,42 +915,32 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_block_kernel(PrefillA
     float M = -INFINITY, L = 0.0f;
     {
         v4f own[MT], os[MT];
-        float om, ol;
         const int at = half * 4 + wave, from = (1 - half) * 4 + wave;
-        if (BOTH || half == 1) {
 #pragma unroll
-            for (int m = 0; m < MT; m++)
-                ob[(at * MT + m) * 64 + lane] = BOTH && half == 0 ? st.o[m][NJ - 1] : st.o[m][0];
-            mb[(at * 64 + lane) * 2] = BOTH && half == 0 ? st.mrow[NJ - 1] : st.mrow[0];
-            mb[(at * 64 + lane) * 2 + 1] = BOTH && half == 0 ? lrow[NJ - 1] : lrow[0];
-        }
-        const bool last = BOTH && half == 1;   // this half keeps its last row tile
+        for (int m = 0; m < MT; m++) ob[(at * MT + m) * 64 + lane] = half == 0 ? st.o[m][1] : st.o[m][0];
+        mb[(at * 64 + lane) * 2] = half == 0 ? st.mrow[1] : st.mrow[0];
+        mb[(at * 64 + lane) * 2 + 1] = half == 0 ? lrow[1] : lrow[0];
 #pragma unroll
         for (int m = 0; m < MT; m++) {
             acc[m] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-            own[m] = last ? st.o[m][NJ - 1] : st.o[m][0];
+            own[m] = half == 1 ? st.o[m][1] : st.o[m][0];
         }
-        const float mo = last ? st.mrow[NJ - 1] : st.mrow[0], lo = last ? lrow[NJ - 1] : lrow[0];
+        const float mo = half == 1 ? st.mrow[1] : st.mrow[0], lo = half == 1 ? lrow[1] : lrow[0];
         __syncthreads();
-        if (!BOTH && half == 1 && segs == 1) return;
-        if (BOTH || half == 0) {
 #pragma unroll
-            for (int m = 0; m < MT; m++) os[m] = ob[(from * MT + m) * 64 + lane];
-            om = mb[(from * 64 + lane) * 2];
-            ol = mb[(from * 64 + lane) * 2 + 1];
-            if (half == 0) {
-                merge_part<MT>(M, L, acc, mo, lo, own);
-                merge_part<MT>(M, L, acc, om, ol, os);
-            } else {
-                merge_part<MT>(M, L, acc, om, ol, os);
-                merge_part<MT>(M, L, acc, mo, lo, own);
-            }
+        for (int m = 0; m < MT; m++) os[m] = ob[(from * MT + m) * 64 + lane];
+        const float om = mb[(from * 64 + lane) * 2], ol = mb[(from * 64 + lane) * 2 + 1];
+        if (half == 0) {
+            merge_part<MT>(M, L, acc, mo, lo, own);
+            merge_part<MT>(M, L, acc, om, ol, os);
+        } else {
+            merge_part<MT>(M, L, acc, om, ol, os);
+            merge_part<MT>(M, L, acc, mo, lo, own);
         }
     }
-    const bool mine_rows = BOTH || half == 0;
-    const int tile = wave * NJ + (BOTH ? half : 0);   // the row tile this wave finishes
+    const int tile = wave * NJ + half;   // the row tile this wave finishes
     if (segs == 1) {
-        store_rows<HD, G, NJ>(a, kvh, i0, tile, lane, acc, L);
+        store_rows<HD, G>(a, kvh, i0, tile, lane, acc, L);
         return;
     }
 
@@ -961,23 +951,21 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_block_kernel(PrefillA
         __builtin_amdgcn_make_buffer_rsrc(a.partials + pblock * S::RW * PS, 0, segs * S::RW * PS * 4, 0x00020000);
     int *counter = a.counters + ((size_t)kvh * a.qblocks + blk) * kCounterStrideP;
     const int r = tile * 16 + l16;
-    if (mine_rows) {
-        const int base = (sp * S::RW + r) * PS;
+    const int base = (sp * S::RW + r) * PS;
 #pragma unroll
-        for (int m = 0; m < MT; m++)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[m]), prs, (base + m * 16 + 4 * lg) * 4,
-                                                   0, kCoherentP);
-        if (lg == 0) {
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(M), prs, (base + HD) * 4, 0, kCoherentP);
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(L), prs, (base + HD + 1) * 4, 0, kCoherentP);
-        }
+    for (int m = 0; m < MT; m++)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[m]), prs, (base + m * 16 + 4 * lg) * 4, 0,
+                                               kCoherentP);
+    if (lg == 0) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(M), prs, (base + HD) * 4, 0, kCoherentP);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(L), prs, (base + HD + 1) * 4, 0, kCoherentP);
     }
     __builtin_amdgcn_s_waitcnt(0);   // this thread's partial is at the point of coherence
     int *flag = reinterpret_cast<int *>(&tiles[0][0]);
     __syncthreads();                 // every thread's partial; every wave done with the exchanged rows
     if (tid == 0) *flag = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == segs - 1;
     __syncthreads();
-    if (!*flag || !mine_rows) return;
+    if (!*flag) return;
     if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
     // the runs' partials, the next one's loads in flight while one is merged
@@ -1008,22 +996,11 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_block_kernel(PrefillA
         if (s2 + 2 < segs) load(s2 + 2, os[0], ms[0], ls[0]);
         if (s2 + 1 < segs) fold(s2 + 1, os[1], ms[1], ls[1]);
     }
-    store_rows<HD, G, NJ>(a, kvh, i0, tile, lane, acc2, L2);
+    store_rows<HD, G>(a, kvh, i0, tile, lane, acc2, L2);
 }
 
-// Rows per work-group: 128 (two row tiles per wave) by default;
-// TQ_HIP_PREFILL_ROWS=64 selects one row tile per wave where G allows.
-int prefill_rows(int g) {
-    static int forced = [] {
-        const char *s = getenv("TQ_HIP_PREFILL_ROWS");
-        return s ? atoi(s) : 0;
-    }();
-    if (g == 8) return 128;
-    return forced == 64 ? 64 : 128;
-}
-
-// Query tokens per work-group for a shape (the kernel's QB).
-int prefill_qb(int g) { return 64 * (prefill_rows(g) == 128 ? 2 : 1) / g; }
+// Query tokens per work-group for a group size (the kernel's QB).
+int prefill_qb(int g) { return 64 * NJ / g; }
 
 // TQ_HIP_PREFILL_WHOLE=1 keeps every block one run, =0 cuts every block into
 // as many runs as the plan may (tests of both at any size); read on every
@@ -1033,13 +1010,13 @@ int prefill_whole_env() {
     return (s && *s) ? (s[0] == '1' ? 1 : 0) : -1;
 }
 struct PrefillPlan {
-    int qblocks, whole, chunk, nsp, rows, items;
+    int qblocks, whole, chunk, nsp, items;
 };
 PrefillPlan plan_prefill(int hd, int g, int n_kv_heads, int pos0, int n) {
     const int qb = prefill_qb(g);
     const int qblocks = (n + qb - 1) / qb;
     const RunPlan r = plan_runs(hd, qb, n_kv_heads, pos0, n, qblocks, prefill_whole_env());
-    return PrefillPlan{qblocks, r.whole, r.chunk, r.runs, 64 * (prefill_rows(g) == 128 ? 2 : 1), r.items};
+    return PrefillPlan{qblocks, r.whole, r.chunk, r.runs, r.items};
 }
 
 // Byte offset of the staged q blocks in the image buffer (after the key
@@ -1051,7 +1028,7 @@ size_t qimg_offset(int head_dim, int n_kv_heads, int kend) {
 }
 
 // The staging launch (key tiles and q blocks), then the attention.
-template <int HD, int G, int NJ>
+template <int HD, int G>
 hipError_t launch_hd_g(const TqPrefillArgs &t, const PrefillArgs &a, int items, hipStream_t s) {
     StageArgs st;
     st.view = t.view;
@@ -1074,22 +1051,21 @@ hipError_t launch_hd_g(const TqPrefillArgs &t, const PrefillArgs &a, int items, 
     st.q_norm = t.q_norm;
     st.k_norm = t.k_norm;
     st.rms_eps = t.rms_eps;
-    hipLaunchKernelGGL((prefill_stage_kernel<HD, G, NJ>), dim3(a.n_tiles + a.qblocks, t.n_kv_heads), dim3(kThreads),
+    hipLaunchKernelGGL((prefill_stage_kernel<HD, G>), dim3(a.n_tiles + a.qblocks, t.n_kv_heads), dim3(kThreads),
                        0, s, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((prefill_block_kernel<HD, G, NJ>), dim3(items * t.n_kv_heads), dim3(2 * kThreads), 0, s, a);
+    hipLaunchKernelGGL((prefill_block_kernel<HD, G>), dim3(items * t.n_kv_heads), dim3(2 * kThreads), 0, s, a);
     return hipGetLastError();
 }
 
 template <int HD>
 hipError_t launch_hd(const TqPrefillArgs &t, const PrefillArgs &a, int g, int items, hipStream_t s) {
-    const bool wide = prefill_rows(g) == 128;
     switch (g) {
-        case 1: return wide ? launch_hd_g<HD, 1, 2>(t, a, items, s) : launch_hd_g<HD, 1, 1>(t, a, items, s);
-        case 2: return wide ? launch_hd_g<HD, 2, 2>(t, a, items, s) : launch_hd_g<HD, 2, 1>(t, a, items, s);
-        case 4: return wide ? launch_hd_g<HD, 4, 2>(t, a, items, s) : launch_hd_g<HD, 4, 1>(t, a, items, s);
-        case 8: return launch_hd_g<HD, 8, 2>(t, a, items, s);
+        case 1: return launch_hd_g<HD, 1>(t, a, items, s);
+        case 2: return launch_hd_g<HD, 2>(t, a, items, s);
+        case 4: return launch_hd_g<HD, 4>(t, a, items, s);
+        case 8: return launch_hd_g<HD, 8>(t, a, items, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1110,14 +1086,14 @@ void tq_prefill_scratch(int head_dim, int group, int n_kv_heads, int pos0, int n
         *counter_ints = 0;
         return;
     }
-    *partial_bytes = (size_t)n_kv_heads * p.qblocks * p.nsp * p.rows * (head_dim + 4) * sizeof(float);
+    *partial_bytes = (size_t)n_kv_heads * p.qblocks * p.nsp * (64 * NJ) * (head_dim + 4) * sizeof(float);
     *counter_ints = (size_t)n_kv_heads * p.qblocks * kCounterStrideP;
 }
 
 size_t tq_prefill_image_bytes(int head_dim, int group, int n_kv_heads, int pos0, int n) {
     const PrefillPlan p = plan_prefill(head_dim, group, n_kv_heads, pos0, n);
-    const size_t qrow = head_dim == 64 ? PShape<64, 1, 1>::QCS + 2 * 4 : PShape<128, 1, 1>::QCS + 4 * 4;
-    return qimg_offset(head_dim, n_kv_heads, pos0 + n) + (size_t)n_kv_heads * p.qblocks * p.rows * qrow;
+    const size_t qrow = head_dim == 64 ? PShape<64, 1>::QCS + 2 * 4 : PShape<128, 1>::QCS + 4 * 4;
+    return qimg_offset(head_dim, n_kv_heads, pos0 + n) + (size_t)n_kv_heads * p.qblocks * (64 * NJ) * qrow;
 }
 
 hipError_t tq_launch_prefill(const TqPrefillArgs &t, hipStream_t s) {

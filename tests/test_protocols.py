@@ -2,7 +2,7 @@
 every interleaving of a few work-groups (exhaustive for small counts,
 randomised for larger ones).  They check the design, not the GPU code:
 
-* split-K combine (decode3.hip, the split prefill kernel in prefill.hip):
+* split-K combine (decode3.hip, the runs of prefill_block_kernel):
   every work-group stores its partial (o, m, l), waits for the stores, then
   adds one to its head's arrival counter; the one that reads n-1 resets the
   counter and merges all partials in split order, its own from registers.
@@ -10,9 +10,10 @@ randomised for larger ones).  They check the design, not the GPU code:
   exactly one work-group merges; the counter is 0 again after the launch, so
   the next launch starts clean; the merged bytes do not depend on the order
   of arrival.
-* the whole-block prefill merge (prefill_block_kernel): two halves, a barrier,
-  half 1's rows in LDS, half 0 merges in half order: the same merge, fixed
-  order.
+* the prefill's exchange of halves (prefill_block_kernel): each of two halves
+  holds both row tiles of a wave over its own key tiles; half h leaves row tile
+  1 - h in LDS, a barrier, then finishes row tile h from its own and the one it
+  finds, in half order.
 
 The merge arithmetic is the kernels' (exp2 of the difference to the running
 max, fp32 throughout); a planted mistake (merging in arrival order) makes
@@ -129,13 +130,56 @@ def test_consecutive_launches_start_clean():
         assert res.tobytes() == merge(parts, range(n)).tobytes()
 
 
-def test_whole_block_two_halves():
-    """prefill_block_kernel: half 0 merges its rows with half 1's in half
-    order; a half with no key (the one-tile block) leaves half 0's rows
-    exactly as they were."""
+def exchange(st, order, wrong_tile=False):
+    """Two halves' (m, l, o) of row tiles 0 and 1, st[half][tile]: the LDS
+    exchange with the halves' steps run in `order`, a barrier between the
+    stores and the merges.  Returns the finished row tiles."""
+    lds, out = {}, {}
+    for half in order:
+        lds[half] = st[half][half if wrong_tile else 1 - half]   # the tile the other one finishes
+    for half in order:
+        own, other = st[half][half], lds[1 - half]
+        out[half] = merge([own, other], [0, 1] if half == 0 else [1, 0])
+    return out
+
+
+def exact_tiles(st):
+    """The merged row tiles in fp64, and the bound of the fp32 merge: factors,
+    products, sums and the quotient are each rounded once, a few 2^-24 of the
+    terms."""
+    for tile in (0, 1):
+        m = np.array([st[h][tile][0] for h in (0, 1)], np.float64)
+        w = np.exp2(m - m.max())
+        den = sum(w[h] * float(st[h][tile][1]) for h in (0, 1))
+        o = [st[h][tile][2].astype(np.float64) for h in (0, 1)]
+        yield (w[0] * o[0] + w[1] * o[1]) / den, 8 * 2.0 ** -24 * (w[0] * np.abs(o[0]) + w[1] * np.abs(o[1])) / den
+
+
+EMPTY = (np.float32(-np.inf), np.float32(0.0), np.zeros(8, np.float32))
+
+
+def test_halves_exchange_row_tiles():
+    """Every row tile is finished once, with both halves' parts of that tile in
+    half order, whichever half is first; a half with no key (a run of one tile)
+    leaves the other's rows exactly as they were."""
     rng = np.random.default_rng(9)
-    h0, h1 = random_parts(rng, 2)
-    assert merge([h0, h1], [0, 1]).tobytes() == merge([h0, h1], [0, 1]).tobytes()
-    empty = (np.float32(-np.inf), np.float32(0.0), np.zeros(8, np.float32))
-    alone = merge([h0, empty], [0, 1])
-    assert alone.tobytes() == (h0[2] / h0[1]).astype(np.float32).tobytes()
+    for _ in range(20):
+        st = [random_parts(rng, 2), random_parts(rng, 2)]
+        out = exchange(st, [0, 1])
+        for tile, (exact, bound) in enumerate(exact_tiles(st)):
+            assert (np.abs(out[tile] - exact) <= bound).all()
+        again = exchange(st, [1, 0])
+        assert all(again[t].tobytes() == out[t].tobytes() for t in (0, 1))
+        lone = exchange([st[0], [EMPTY, EMPTY]], [0, 1])
+        for tile in (0, 1):
+            m, l, o = st[0][tile]
+            assert lone[tile].tobytes() == (o / l).astype(np.float32).tobytes()
+
+
+def test_planted_wrong_tile_is_caught():
+    """A half that leaves the row tile it finishes itself: beyond the bound."""
+    rng = np.random.default_rng(10)
+    st = [random_parts(rng, 2), random_parts(rng, 2)]
+    out = exchange(st, [0, 1], wrong_tile=True)
+    for tile, (exact, bound) in enumerate(exact_tiles(st)):
+        assert not (np.abs(out[tile] - exact) <= bound).all()
