@@ -44,6 +44,9 @@ def rel_l2(a, b) -> float:
     return float(np.sqrt(((a - b) ** 2).sum() / max((b * b).sum(), 1e-300)))
 
 
+REF_DIR = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle", "_ref")
+
+
 @pytest.fixture(scope="module")
 def nat():
     from tailorquantkernel_amd import native
@@ -54,8 +57,8 @@ def nat():
 
 def dropin(variant):
     if not Ref.available(dropin=variant):
-        if not os.path.exists("/root/reference/model/attention_layer.c"):
-            pytest.skip("the drop-in build needs the reference's sources")
+        if os.path.exists(os.path.join(REF_DIR, "ABSENT")):
+            pytest.skip("the last build had none of the reference's sources (oracle/_ref/ABSENT)")
         pytest.fail(f"oracle/_ref/{Ref._name(True, variant)} is missing: build it with `make -C oracle dropin`")
     return Ref(dropin=variant)
 

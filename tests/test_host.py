@@ -245,3 +245,17 @@ def test_dev_model_guards(attn):
     assert L.tq_dev_forward_batch(C.byref(ctx), C.byref(ws), toks, 2, 1) == -1
     assert L.tq_dev_prefill(None, toks, 2) == -1
     assert L.tq_dev_prefill(C.byref(ctx), toks, 2) == -1
+
+
+def test_missing_dropin_library_skips_only_where_the_build_recorded_it(monkeypatch, tmp_path):
+    """The drop-in tests skip where the last build noted that the reference's
+    sources were absent; a library missing for any other reason fails them."""
+    from oracle.binding import Ref
+    from tests import test_gpu_dropin
+    monkeypatch.setattr(Ref, "available", staticmethod(lambda scalar=False, dropin=None: False))
+    monkeypatch.setattr(test_gpu_dropin, "REF_DIR", str(tmp_path), raising=False)
+    for outcome in (pytest.fail.Exception, pytest.skip.Exception):
+        with pytest.raises((pytest.fail.Exception, pytest.skip.Exception)) as raised:
+            test_gpu_dropin.dropin("fused")
+        assert raised.type is outcome
+        (tmp_path / "ABSENT").write_text("no sources\n")
