@@ -222,8 +222,8 @@ __device__ __forceinline__ void dma4(const void *src, unsigned char *dst) {
 
 // The same copies from a uniform base plus a 32-bit lane offset (the saddr
 // form) to LDS byte address lds + IMM: no per-lane 64-bit address arithmetic,
-// and two scalar instructions with the copy (M0 is left changed; nothing else
-// in these kernels uses it).  base and lds are uniform.
+// and two scalar instructions with the copy, the s_nop among them (M0 is left
+// changed; nothing else in these kernels uses it).  base and lds are uniform.
 template <int IMM>
 __device__ __forceinline__ void dma16s(const unsigned char *base, uint32_t off, uint32_t lds) {
     asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
@@ -504,10 +504,10 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v32f __attribute__((ext_vector_type(32)));
 
 // BX4: the activation rows are 16-byte aligned and nb % 4 == 0.
-// Q4: tiled Q4 matrices.  A holds [4 blocks][128 rows][16 B] nibble bytes (one
-// copy per thread instead of two); each lane turns its 8 bytes into 16 x its
-// 8 codes (low nibbles for k < 16, high for k >= 16), and the int32 products
-// are shifted back by 4 before scaling.
+// Q4: tiled Q4 matrices.  A holds [128 rows][4 slots][16 B] nibble bytes (one
+// copy per thread instead of two); each lane turns its row's 16 bytes of a block
+// into 16 x its 16 codes (low nibbles for k < 16, high for k >= 16), and the
+// scales are 1/16 of the matrix's.
 template <bool BX4, bool Q4, bool UNI, bool XS, int TT>
 __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
     static_assert(!UNI || BX4, "uniform copies need whole 16-byte stages");
@@ -745,7 +745,7 @@ __global__ __launch_bounds__(512, BX4 ? 4 : 2) void gemm_q8_kernel(GemvArgs a) {
 #pragma unroll
     for (int t2 = 0; t2 < T2; t2++) acc[t2] = v16f(0.0f);
 
-    // Two buffers (73.7 KB, so two work-groups share a CU): stage st+1 is
+    // Two buffers (74.8 KB, or 56.3 with 64 tokens: two work-groups share a CU): stage st+1 is
     // copied while stage st is multiplied.
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_u8 *)smem;
     if constexpr (uni) {

@@ -549,11 +549,10 @@ def test_prefill(nat, oracle, shape):
 @pytest.mark.parametrize("whole", ["1", "0"])
 @pytest.mark.parametrize("shape", PREFILL_SHAPES[:8])
 def test_prefill_both_plans(nat, oracle, shape, whole, monkeypatch):
-    """The dense shapes through each of the two attention kernels, forced:
-    whole query blocks (one 8-wave work-group per block, its two halves merged
-    in LDS) and the paired, split blocks (partials merged by the last
-    segment).  Both against the oracle's sequential steps, cache bytes
-    bit-exact."""
+    """The dense shapes with every query block one run (one 8-wave work-group
+    per block, its two halves merged in LDS) and with every block cut into as
+    many runs as may be (partials merged by the last to arrive).  Both against
+    the oracle's sequential steps, cache bytes bit-exact."""
     monkeypatch.setenv("TQ_HIP_PREFILL_WHOLE", whole)
     check_prefill(nat, oracle, shape)
 
