@@ -1091,26 +1091,17 @@ long gemm_wgs(int rows, int n_tok, int toks) {
 
 // Tokens per tile of a launch over n_tok: 64 where one such tile holds them,
 // and up to 320 tokens where 128-token tiles would be half padding at the end
-// (an odd count of 64s; a 64-token tile takes 0.54 of a 128-token one).  8B
-// MLP, us with 64 / 128, Q8 then Q4: 130 tokens 140 / 155, 131 / 150; 190: 142
-// / 155, 135 / 154; 300: 206 / 225, 206 / 224.  At 420 the gain is gone (277 /
-// 282, 283 / 277) and at 550 it is a loss (371 / 345).
-//
-// Five tiles of 64 against three of 128 lose where they alone give every CU a
-// work-group and so end the K splits (`split`: the launch may split) that three
-// leave room for: 7,169 to 10,240 rows.  MLP over 320 tokens, us with 64 / 128, Q8
-// then Q4: 8,192 x 28,672 809 / 789, 818 / 786; 7,168 x 4,096 135 / 133, 151 /
-// 136; 8,192 x 5,120 163 / 168, 175 / 171.  (Three of 64 against two do not
-// lose so: 4,096 x 7,168 over 160 tokens 80 / 86, 85 / 87.)
+// (an odd count of 64s; a 64-token tile takes 0.54 of a 128-token one).  No
+// bit depends on it: the K splits do not follow the tile (gemm_ksplit).  MLP,
+// us with 64 / 128, Q8 then Q4: 4,096 x 14,336 over 129 tokens 124 / 139, 126 / 141,
+// 300: 204 / 207, 212 / 210; 8,192 x 28,672, 300: 740 / 823, 722 / 814; 2,048 x 5,632,
+// 300: 59 / 73, 61 / 77; 8,192 x 5,120, 300: 164 / 161, 173 / 167 (400 tiles of 10,240
+// rows in two splits, 1.6 rounds of the CUs, against 0.9).  Choosing by whole
+// rounds lost more than it gained (129 tokens 139 again).  At 420 tokens of 4,096 x
+// 14,336 the gain was gone (277 / 282, 283 / 277) and at 550 a loss (371 / 345).
 constexpr int kGemmSmallToks = 320;
-constexpr int kSplitWgs = 512;
 
-int gemm_toks(int rows, int n_tok, bool split) {
-    if (n_tok <= 64) return 64;
-    if (n_tok > kGemmSmallToks || (n_tok + 63) / 64 % 2 == 0) return 128;
-    const bool ends_splits = gemm_wgs(rows, n_tok, 64) >= kSplitWgs / 2 && gemm_wgs(rows, n_tok, 128) < kSplitWgs / 2;
-    return split && n_tok > 192 && ends_splits ? 128 : 64;
-}
+int gemm_toks(int n_tok) { return n_tok <= 64 || (n_tok <= kGemmSmallToks && (n_tok + 63) / 64 % 2) ? 64 : 128; }
 
 template <int TT>
 hipError_t launch_gemm_t(const GemvArgs &u, bool bx4, unsigned grid, hipStream_t s) {
@@ -1156,7 +1147,7 @@ hipError_t launch_gemm_t(const GemvArgs &u, bool bx4, unsigned grid, hipStream_t
 }
 
 hipError_t launch_gemm(const GemvArgs &a, int ksplit, hipStream_t s) {
-    const int toks = gemm_toks(a.rows_total, a.n_tok, ksplit > 1);
+    const int toks = gemm_toks(a.n_tok);
     const long grid = gemm_wgs(a.rows_total, a.n_tok, toks) * ksplit;
     if (grid > INT32_MAX) return hipErrorInvalidValue;
     const bool bx4 = (((uintptr_t)a.xq & 15) == 0) && a.nb % kGemmKB == 0;
@@ -1194,18 +1185,24 @@ hipError_t launch_gemm(const GemvArgs &a, int ksplit, hipStream_t s) {
 
 // Split-K GEMM while the tiles alone leave CUs of the 256 idle (each tile
 // then runs the whole K loop): K is cut into S runs of stages, as many as
-// keep the grid within one round of 512 work-groups (two per CU), each split
-// writing a partial tile that one more launch sums in split order.  MLP at
-// the 8B shape, us with Q8 / Q4 weights over 16, 64, 100, 256 rows: 74 / 58,
-// 84 / 70, 106 / 98, 158 / 154; before 64-token tiles 96 / 88, 105 / 97,
-// 114 / 105, 164 / 157.  The least is 16 tokens, as without a workspace: up to
-// 15 a row's bits are the GEMV's whatever its batch.  (Splits from 9 tokens
-// took 72 / 59 for 100 / 76 us of GEMV launches there, with other bits.)
+// keep a grid of 128-token tiles within one round of 512 work-groups (two per
+// CU), each split writing a partial tile that one more launch sums in split
+// order.  S is counted in 128-token tiles whatever the tile is, so that a row's
+// bits and the length of its sums do not change with the padding.  With S from
+// the 64-token tiles (fewer and longer sums; 300 rows of 4,096 x 14,336 203 for 214
+// us, of 8,192 x 28,672 816 for 794) an attention layer over 300 tokens was 4.29e-4
+// from a 64-bit evaluation over 48 seeds, and is 4.16e-4.  MLP at the 8B shape, us with Q8 / Q4 weights over 16, 64, 100, 256
+// rows: 63 / 56, 71 / 63, 94 / 93, 144 / 145; with 16 x 16 products and only
+// 128-token tiles 112 / 109, 131 / 126, 144 / 139, 197 / 207.  The least is 16
+// tokens, as without a workspace: up to 15 a row's bits are the GEMV's whatever
+// its batch.  (Splits from 9 tokens took 62 / 56 for 90 / 75 us of GEMV launches
+// there, with other bits.)
+constexpr int kSplitWgs = 512;
 constexpr int kSplitMinTokens = 16;
 
 int gemm_ksplit(int rows, int cols, int n_tok) {
     if (n_tok < kSplitMinTokens) return 1;
-    const long wgs = gemm_wgs(rows, n_tok, gemm_toks(rows, n_tok, true));
+    const long wgs = gemm_wgs(rows, n_tok, 128);
     // once every CU holds a tile, splitting adds occupancy but not CUs, and
     // the partials' traffic outweighs it (4,096 x 14,336 at 1,024 tokens)
     if (wgs >= kSplitWgs / 2) return 1;

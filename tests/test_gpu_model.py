@@ -251,44 +251,6 @@ def test_mlp_layer_split_fused(nat, oracle, fmt, hidden, inter, n, monkeypatch):
     assert mlp(rows_bytes)[0] == nat.EINVAL and mlp(wsb - 256)[0] == nat.EINVAL
 
 
-@pytest.mark.parametrize("fmt,n", [("q8", 257), ("q8", 320), ("q4", 320)])
-def test_mlp_layer_keeps_splits_at_five_tiles(nat, oracle, fmt, n):
-    """257-320 rows of a matrix where five 64-token tiles per row tile would
-    give every CU a work-group and end the K splits: three 128-token tiles,
-    split in two (both splits' partials of the down matmul, past the room of
-    the gate/up ones, lose the pattern written before), within the matmul bar
-    of the oracle's down projection of the hidden rows."""
-    lib = nat.load()
-    hidden, inter = 7296, 256
-    rng = np.random.default_rng(n)
-    q4 = fmt == "q4"
-    pack = oracle.pack_matrix_q4 if q4 else oracle.pack_matrix_q8
-    wg, wu, wd = (pack(rng.standard_normal((r, c)).astype(np.float32) * 0.1)
-                  for r, c in ((inter, hidden), (inter, hidden), (hidden, inter)))
-    mats = [tiled(nat, wg, inter, hidden), tiled(nat, wu, inter, hidden), tiled(nat, wd, hidden, inter)]
-    w = nat.MlpWeights(*(m.ptr for m in mats), hidden, inter, nat.FORMAT_Q4 if q4 else nat.FORMAT_Q8)
-    wsb = lib.tq_hip_mlp_ws_bytes(C.byref(w), n)
-    ws = nat.DeviceBuffer(wsb)
-    ws.upload(np.full(wsb, 0xA5, np.uint8))
-    dx, dout = dev(nat, normal(n * hidden, 3) * 2), nat.DeviceBuffer(n * hidden * 4)
-    nat.check(lib.tq_hip_mlp_layer_async(C.byref(w), n, dx.ptr, dout.ptr, ws.ptr, wsb, None), "mlp")
-    sync(nat)
-    raw, out = ws.download((wsb,), np.uint8), dout.download((n, hidden), np.float32)
-    al = lambda b: (b + 255) & ~255
-    xq = 2 * al(n * inter * 4)
-    part = raw[xq + al(n * hidden // QK * 36):].view(np.uint32)[:2 * n * hidden]
-    assert part.size == 2 * n * hidden and (part != 0xA5A5A5A5).all()
-    nbi = inter // QK
-    codes = raw[xq:xq + n * inter].view(np.int8).reshape(nbi, 2, n, 16)
-    scales = raw[xq + n * inter:xq + n * inter + 4 * n * nbi].view(np.float32).reshape(nbi, n)
-    for t in (0, 63, 64, 127, 128, 255, 256, n - 1):
-        rows = np.zeros(nbi, BLOCK_Q8)
-        rows["d"] = scales[:, t]
-        rows["q"] = codes[:, :, t, :].reshape(nbi, QK)
-        ref = (oracle.matmul_q4 if q4 else oracle.matmul_q8)(wd, rows, hidden, inter, 1)[0]
-        assert rel_l2(out[t], ref) <= 1e-5
-
-
 def random_matrix(nat, rows, cols, seed, q4=False):
     """A tiled matrix on the device of random codes, with scales for weights of about 0.02."""
     rng = np.random.default_rng(seed)
@@ -321,6 +283,27 @@ def test_mlp_rows_up_to_15_are_the_row_alone(nat, fmt, hidden, inter, n):
     assert np.array_equal(mlp(n, 0, roomy).view(np.int32), together.view(np.int32))
     alone = np.concatenate([mlp(1, t, wsb) for t in range(n)])
     assert np.array_equal(alone.view(np.int32), together.view(np.int32))
+
+
+@pytest.mark.parametrize("fmt,n,whole", [("q8", 129, 256), ("q4", 192, 256), ("q8", 257, 384), ("q4", 300, 384),
+                                         ("q8", 320, 384)])
+def test_mlp_splits_do_not_follow_the_tile(nat, fmt, n, whole):
+    """Row counts that take 64-token tiles and the next that fills 128-token
+    ones, with K splits that another tile count would change: the same rows,
+    bit for bit."""
+    lib = nat.load()
+    hidden, inter, q4 = 4096, 2048, fmt == "q4"
+    mats = [random_matrix(nat, r, c, i, q4) for i, (r, c) in enumerate(((inter, hidden), (inter, hidden), (hidden, inter)))]
+    w = nat.MlpWeights(*(m.ptr for m in mats), hidden, inter, nat.FORMAT_Q4 if q4 else nat.FORMAT_Q8)
+    wsb = lib.tq_hip_mlp_ws_bytes(C.byref(w), whole)
+    ws = nat.DeviceBuffer(wsb)
+    dx, dout = dev(nat, normal(whole * hidden, 5) * 2), nat.DeviceBuffer(whole * hidden * 4)
+    outs = []
+    for rows in (n, whole):
+        nat.check(lib.tq_hip_mlp_layer_async(C.byref(w), rows, dx.ptr, dout.ptr, ws.ptr, wsb, None), "mlp")
+        sync(nat)
+        outs.append(dout.download((whole, hidden), np.float32)[:n].view(np.int32))
+    assert np.array_equal(*outs)
 
 
 @pytest.mark.parametrize("hidden,inter,n", [(512, 1024, 16), (512, 1024, 20), (512, 1024, 130), (512, 1024, 300)])
