@@ -1045,32 +1045,27 @@ hipError_t launch_gemv(const GemvArgs &a, int tcap, bool xf, int rw, int gc, hip
     }
 }
 
-// One GEMV launch of up to tmax tokens streams the weights once, at about
-// 5 TB/s of Q8 bytes, plus its launch.  Q4 launches of 8 tokens take as long:
-// their vector work is the same.  Where 8 tokens do not fit, launches of 4 are
-// bound by their own bytes: 4,096 x 14,336 14.4 us, Q4 10.2.
-double gemv_us(int rows, int cols, bool q4, int tmax) {
-    return (double)rows * cols * (kBlockBytes / (double)kQK) / 5.0e6 * (tmax >= 8 ? 1.0 : q4 ? 0.6 : 0.9) + 2.5;
-}
-
 // From how many tokens on (block_q8 input) the unsplit MFMA GEMM runs instead
 // of GEMV launches of tmax tokens each (TQ_HIP_GEMM_MIN_TOKENS overrides).
-// GEMV's cost grows with the token count; the GEMM's first round of 128-row
-// tiles costs its K loop: measured 0.0072 us per column with 64-token tiles
-// and 0.0133 with 128-token ones.  us, GEMM against GEMV launches:
+// The line is a matter of precision, not of time: a GEMV row is 64 short sums
+// in a tree, a GEMM row one chain over its blocks.  Distance from the 64-bit
+// product of the same codes, GEMV / GEMM: 4,096 columns 8.0e-8 / 2.05e-7, 8,192
+// 8.6e-8 / 2.9e-7, 14,336 9.2e-8 / 3.8e-7.  So it stays where an earlier, slower
+// GEMM (0.0183 us per column for its first round of tiles, against 5 TB/s and 2
+// us per GEMV launch) crossed the GEMV launches: 6144 x 4096 from 81 tokens,
+// 28672 x 4096 from 22, 4096 x 14336 from 70.  The present GEMM is ahead from 33,
+// 12 and 30 on (Q4 43), us, GEMM against GEMV:
 //   6144 x 4096    16 tokens 33 / 18    32: 33 / 33    64: 34 / 63    96: 58 / 94
-//   28672 x 4096    8: 48 / 35    12: 48 / 55    32: 48 / 121    96: 68 / 346
+//   28672 x 4096   8: 48 / 35    12: 48 / 55    16: 37 / 53    20: 38 / 75
 //   4096 x 14336   16: 105 / 58   32: 105 / 116  64: 106 / 231   96: 190 / 345
 //   the same, Q4   28: 114 / 75   40: 114 / 106  48: 114 / 126   64: 114 / 164
-// The model puts the crossovers at 33, 16 (the least), 30 and 42.
-int gemm_min_tokens(int rows, int cols, bool q4, int tmax) {
+int gemm_min_tokens(int rows, int cols, int tmax) {
     const int v = env_int("TQ_HIP_GEMM_MIN_TOKENS", 0);
     if (v > 0) return v;
-    const double per_token = gemv_us(rows, cols, q4, tmax) / tmax;
-    const int n64 = (int)((0.0072 * cols + 3.5) / per_token) + 1;
-    if (n64 <= 64) return n64 < 16 ? 16 : n64;   // up to 15 tokens a row's bits are the GEMV's whatever its batch
-    const int n128 = (int)((0.0133 * cols + 3.5) / per_token) + 1;
-    return n128 < 65 ? 65 : (n128 > 256 ? 256 : n128);
+    const double chunk_us = (double)rows * cols * (kBlockBytes / (double)kQK) / 5.0e6 + 2.0;
+    const double gemm_us = 0.0183 * cols + 2.0;
+    const int n = (int)(tmax * gemm_us / chunk_us) + 1;
+    return n < 16 ? 16 : (n > 256 ? 256 : n);   // up to 15 tokens a row's bits are the GEMV's whatever its batch
 }
 
 // Every 128-row tile inside one segment (segment ends on tile boundaries) and
@@ -1220,7 +1215,7 @@ int gemm_plan(const GemvArgs &a, int n_tok) {
     const int ksplit = a.part ? gemm_ksplit(a.rows_total, a.cols, n_tok) : 1;
     if (ksplit > 1 && (size_t)ksplit * n_tok * a.rows_total <= a.part_floats && env_int("TQ_HIP_GEMM_SPLIT", 1) != 0)
         return ksplit;
-    return n_tok >= gemm_min_tokens(a.rows_total, a.cols, a.q4, pick_tokens(a.nb, false)) ? 1 : 0;
+    return n_tok >= gemm_min_tokens(a.rows_total, a.cols, pick_tokens(a.nb, false)) ? 1 : 0;
 }
 
 // Whether the matmul's input should be quantized into the split layout:

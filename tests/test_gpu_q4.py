@@ -257,24 +257,33 @@ def test_q4_mlp_split_k(nat, oracle, split, monkeypatch):
     check_matmul(out, oracle.matmul_q4(wd, hq, hidden, inter, n), wd, hq, hidden, inter, n, "down")
 
 
-def test_q4_wide_rows_stay_with_gemv(nat, monkeypatch):
-    """14,336 columns: GEMV launches hold 4 tokens and a Q4 one takes 0.7 of a
-    Q8 one, so GEMV stays the default up to 40 tokens (its bits, those of the
-    forced route) and the GEMM takes 48."""
-    rows, cols = 4096, 14336
+@pytest.mark.parametrize("rows,cols,gemv,gemm", [(4096, 14336, (16, 48, 69), (70,)), (6144, 4096, (33, 64, 80), (81, 96)),
+                                                  (512, 512, (16, 44), (45, 64))])
+def test_matmul_keeps_gemv_sums_below_the_line(nat, rows, cols, gemv, gemm, monkeypatch):
+    """Without a workspace the batched matmul takes GEMV launches up to the
+    line of gemm_min_tokens (their bits, those of the forced route) and the
+    GEMM from it on.  The GEMV's tree sums are the closer ones to the 64-bit
+    product: rounding errors of sums that grow over nb / 64 blocks and six
+    doublings are within 2^-24 sqrt(7 + nb / 64) of the result in the mean
+    square (a factor 2 allowed), a chain's over nb blocks are not."""
     rng = np.random.default_rng(1)
-    Wq = blocks4(rows * cols // QK)
+    nb = cols // QK
+    Wq = blocks4(rows * nb)
     Wq["d"] = rng.uniform(0.5, 1.5, Wq.size).astype(np.float32) * 0.005
     Wq["q"] = rng.integers(0, 256, Wq["q"].shape, np.uint8)
     M = Matrix4(nat, Wq, rows, cols)
-    xq = np.zeros(48 * cols // QK, BLOCK_Q8)
+    most = max(gemv + gemm)
+    xq = np.zeros(most * nb, BLOCK_Q8)
     xq["d"] = rng.uniform(0.5, 1.5, xq.size).astype(np.float32) * 0.01
     xq["q"] = rng.integers(-127, 128, xq["q"].shape, np.int8)
-    for n, gemv in ((28, True), (40, True), (48, False)):
-        rows_n = xq[:n * cols // QK]
-        y = gpu_matmul4(nat, M, rows_n, n)
+    few = slice(0, 64 * nb)   # 64 rows, exact
+    w = (codes_q4(Wq[few]).astype(np.float64) * Wq["d"][few, None]).reshape(64, cols)
+    x = (xq["q"].astype(np.float64) * xq["d"][:, None]).reshape(most, cols)
+    for n in gemv + gemm:
+        y = gpu_matmul4(nat, M, xq[:n * nb], n)
         monkeypatch.setenv("TQ_HIP_GEMM_MIN_TOKENS", "1000")
-        forced = gpu_matmul4(nat, M, rows_n, n)
+        forced = gpu_matmul4(nat, M, xq[:n * nb], n)
         monkeypatch.delenv("TQ_HIP_GEMM_MIN_TOKENS")
-        assert np.array_equal(y.view(np.int32), forced.view(np.int32)) == gemv, n
-        assert rel_err(y, forced) <= 1e-5, n
+        assert np.array_equal(y.view(np.int32), forced.view(np.int32)) == (n in gemv), n
+        if n in gemv:
+            assert rel_err(y[:, :64], x[:n] @ w.T) <= 2 * 2.0 ** -24 * np.sqrt(7 + nb / 64), n
